@@ -2632,6 +2632,7 @@ int hdnnp_train_gradient(hdnnp_ctx* c, const double* f_ref, double e_ref,
         A.Eref = e_ref;
         A.wE = w_e;
         A.cF = -2.0 * w_f / (3.0 * (double)n);
+        A.cap = std::max(c->maxNeigh, 1);
         hipCheck(launch_train_u(A, s), "train u");
         {
             int const cap = std::max(c->maxNeigh, 1);

@@ -98,6 +98,7 @@ struct TrainArgs
     double* d2;             // n: |F - Fref|^2
     const double* energy;   // device: E of the last evaluation
     double Eref, wE, cF;    // cF = -2 wF / (3N)
+    int cap;                // LDS neighbour capacity per wave
 };
 int train_atoms_per_block();
 int train_atoms_per_grad_block(ElemDesc const& ed);

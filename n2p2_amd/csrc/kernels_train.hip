@@ -71,181 +71,308 @@ __device__ __forceinline__ double scale_slope(ScaleDesc const& s)
             || s.type == ST_SCALESIGMA) ? s.sfac : 1.0;
 }
 
-// u_as for every SF of atom a, and |F_a - Fref_a|^2.  One wave per atom.
+// u_as for every SF of atom a, and |F_a - Fref_a|^2.
+//
+// One wave per atom, organised as the SF kernel (sf_core.h): neighbours
+// staged in LDS partitioned by element, unordered pairs of a group's blocks
+// in diagonal order, passing pairs compacted through an LDS queue so that
+// every lane evaluates one triplet.  Staged per neighbour j, besides the
+// geometry and the cutoff values: e_j = d_a - d_j and t_j = dr_aj . e_j with
+// the residuals d = F - Fref, so that a triplet needs three scalars
+//   t_j, t_k, t_jk = dr_jk . (d_k - d_j) = (dr_ak - dr_aj) . (e_j - e_k).
+// With p1, p2, p3 of SymFncExpAngn.cpp:79-225 / SymFncExpAngw.cpp:79-208 (and
+// SymFncExpAngnWeighted.cpp:79-228) the members' terms contract to
+//   p1 t_j + p2 t_k + p3 t_jk = fg (zeta lambda A + plambda (B - 2 eta C)),
+//   A = pfc ((t_j + t_k + t_jk) / (rij rik) - cos (t_j / rij^2 + t_k / rik^2)),
+//   B = f'c(rij)/rij fc(rik) fc(rjk) t_j + fc(rij) f'c(rik)/rik fc(rjk) t_k
+//     - fc(rij) fc(rik) f'c(rjk)/rjk t_jk               (last term narrow only)
+//   C = pfc ((rij - rs)/rij t_j + (rik - rs)/rik t_k - (rjk - rs)/rjk t_jk),
+// so a member costs its power and three operations, one exponential serves an
+// (eta, rs) run and one power chain a lambda run.
+//
+// Bound by FP64 VALU issue like the SF kernel.  The form before walked the
+// pairs row by row over the whole list (every element pair tested for every
+// group, idle lanes kept) and evaluated exp, pow, square roots and divisions
+// per member: 4.33 ms on a 1,536-atom water box and 3.27 ms on 192 atoms,
+// against 0.131 and 0.103 ms here.
+template <int MAXM, int CT, bool GENPOW>
 __global__ __launch_bounds__(64) void k_train_u(TrainArgs A)
 {
+    extern __shared__ __align__(16) double sm[];
+    __shared__ int sStart[kMaxElements], sCnt[kMaxElements];
+    __shared__ MParam<double> MP[kMaxMembers];
+    int const cap = A.cap;
+    double4* const P = (double4*)sm;        // x, y, z, r
+    double4* const Q = P + cap;             // f_c, 1/r, f_c'/r, t
+    double* const E = (double*)(Q + cap);   // d_a - d_j, x, y, z planes
+    int* const QUEUE = (int*)(E + 3 * cap);
     int const a = blockIdx.x;
-    if (a >= A.n) return;
     int const lane = threadIdx.x;
     ModelTables const& T = A.T;
-    int const e = A.elem[a];
-    ElemDesc const& ed = T.elem[e];
+    int const ne = T.ne;
+    ElemDesc const& ed = T.elem[A.elem[a]];
     double da[3];
     for (int k = 0; k < 3; ++k)
         da[k] = A.F[3 * (size_t)a + k] - A.Fref[3 * (size_t)a + k];
     if (lane == 0) A.d2[a] = da[0] * da[0] + da[1] * da[1] + da[2] * da[2];
     double* __restrict__ U = A.U + (size_t)a * A.ldG;
-    int const o = A.off[a], m = A.cnt[a];
-    for (int gi = ed.g0; gi < ed.g0 + ed.nrad; ++gi)
+    int const s0 = A.off[a], n = A.cnt[a];
     {
-        GroupDesc const g = T.group[gi];
-        CutCfg const cc = T.cfg[ed.cfg0 + g.cfg];
-        MemberDesc const* __restrict__ mem = T.member + g.mem0;
-        bool const weighted = sf_weighted(g.type);
-        double acc[kMaxMembers];
+        int start[kMaxElements];
 #pragma unroll
-        for (int q = 0; q < kMaxMembers; ++q) acc[q] = 0.0;
-        for (int t = lane; t < m; t += 64)
+        for (int q = 0; q < kMaxElements; ++q) start[q] = 0;
+        for (int base = 0; base < n; base += 64)
         {
-            int const j = A.nbrJ[o + t];
-            if (!weighted && A.elem[j] != g.e1) continue;
-            double4 const gq = A.geo[o + t];
-            double const r = gq.w;
-            if (!(r < g.rc)) continue;
-            double fc, dfc;
-            cutoff_fdf<double>(cc, r, fc, dfc);
-            if (weighted)
-            {
-                // SymGrpExpRadWeighted: every term times Z_j.
-                fc *= T.zw[A.elem[j]];
-                dfc *= T.zw[A.elem[j]];
-            }
-            double proj = 0.0;
-            proj += gq.x * (da[0] - (A.F[3 * (size_t)j] - A.Fref[3 * (size_t)j]));
-            proj += gq.y * (da[1] - (A.F[3 * (size_t)j + 1]
-                                     - A.Fref[3 * (size_t)j + 1]));
-            proj += gq.z * (da[2] - (A.F[3 * (size_t)j + 2]
-                                     - A.Fref[3 * (size_t)j + 2]));
-            proj /= r;
+            int const s = base + lane;
+            int const e = s < n ? A.elem[A.nbrJ[s0 + s]] : -1;
 #pragma unroll
-            for (int q = 0; q < kMaxMembers; ++q)
-                if (q < g.nmem)
-                {
-                    double const eta = mem[q].eta, x = r - mem[q].rs;
-                    double const ex = exp(-eta * x * x);
-                    acc[q] += (dfc - 2.0 * eta * x * fc) * ex * proj;
-                }
+            for (int q = 0; q < kMaxElements; ++q)
+                if (q < ne) start[q] += __popcll(__ballot(e == q));
         }
+        int acc = 0;
 #pragma unroll
-        for (int q = 0; q < kMaxMembers; ++q)
-            if (q < g.nmem)
+        for (int q = 0; q < kMaxElements; ++q)
+        {
+            int const c = q < ne ? start[q] : 0;
+            if (lane == 0)
             {
-                double const s = wave_sum(acc[q]);
-                int const sf = mem[q].sf;
-                if (lane == 0)
-                    U[sf] = A.cF * scale_slope(T.scale[ed.sf0 + sf]) * s;
+                sStart[q] = acc;
+                sCnt[q] = c;
             }
+            start[q] = acc;
+            acc += c;
+        }
+        for (int base = 0; base < n; base += 64)
+        {
+            int const s = base + lane;
+            int e = -1, j = 0;
+            double4 g = make_double4(0, 0, 0, 1);
+            if (s < n)
+            {
+                j = A.nbrJ[s0 + s];
+                e = A.elem[j];
+                g = A.geo[s0 + s];
+            }
+            int pos = 0;
+#pragma unroll
+            for (int q = 0; q < kMaxElements; ++q)
+                if (q < ne)
+                {
+                    uint64_t const mask = __ballot(e == q);
+                    if (e == q) pos = start[q] + lanes_below(mask);
+                    start[q] += __popcll(mask);
+                }
+            if (s < n)
+            {
+                double ej[3];
+                for (int k = 0; k < 3; ++k)
+                    ej[k] = da[k] - (A.F[3 * (size_t)j + k]
+                                     - A.Fref[3 * (size_t)j + k]);
+                P[pos] = g;
+                Q[pos] = make_double4(0.0, 1.0 / g.w, 0.0,
+                                      g.x * ej[0] + g.y * ej[1] + g.z * ej[2]);
+                E[pos] = ej[0];
+                E[cap + pos] = ej[1];
+                E[2 * cap + pos] = ej[2];
+            }
+        }
     }
-    // Angular groups, G3 (SymFncExpAngn.cpp:79-225), G9
-    // (SymFncExpAngw.cpp:79-208) and the weighted G3 (type 13,
-    // SymFncExpAngnWeighted.cpp:79-228, every pair of the list):
-    // for the pair (j, k), j < k in list order,
-    // the reference's p1, p2, p3 give
-    //   sum_i d_i . dG/dr_i = p1 dr_ij.(d_a - d_j) + p2 dr_ik.(d_a - d_k)
-    //                       + p3 dr_jk.(d_k - d_j),   dr_jk = dr_ik - dr_ij.
-    for (int gi = ed.g0 + ed.nrad; gi < ed.g0 + ed.ng; ++gi)
+    __syncthreads();
+    int keyCached = -1;
+    for (int gi = ed.g0; gi < ed.g0 + ed.ng; ++gi)
     {
         GroupDesc const g = T.group[gi];
-        CutCfg const cc = T.cfg[ed.cfg0 + g.cfg];
+        int const cfg = ed.cfg0 + g.cfg;
+        CutCfg const cc = T.cfg[cfg];
         MemberDesc const* __restrict__ mem = T.member + g.mem0;
-        bool const wide = g.type == 9;
+        int const nmem = g.nmem;
         bool const weighted = sf_weighted(g.type);
-        double acc[kMaxMembers];
-#pragma unroll
-        for (int q = 0; q < kMaxMembers; ++q) acc[q] = 0.0;
-        for (int j = 0; j + 1 < m; ++j)
+        int const key = 2 * cfg + (weighted ? 1 : 0);
+        if (lane < nmem) MP[lane] = make_mparam<double>(mem[lane], 0.0);
+        if (key != keyCached)
         {
-            int const aj = A.nbrJ[o + j];
-            int const ej = A.elem[aj];
-            double4 const gj = A.geo[o + j];
-            double const rij = gj.w;
-            if (!((weighted || ej == g.e1 || ej == g.e2) && rij < g.rc))
-                continue;
-            double fcij, dfcij;
-            cutoff_fdf<double>(cc, rij, fcij, dfcij);
-            double dj[3];
-            dj[0] = A.F[3 * (size_t)aj] - A.Fref[3 * (size_t)aj];
-            dj[1] = A.F[3 * (size_t)aj + 1] - A.Fref[3 * (size_t)aj + 1];
-            dj[2] = A.F[3 * (size_t)aj + 2] - A.Fref[3 * (size_t)aj + 2];
-            for (int k = j + 1 + lane; k < m; k += 64)
+            // Weighted types: both values times Z_j, so radial terms carry
+            // Z_j and triplet products Z_j Z_k
+            // (SymGrpExpAngnWeighted.cpp:263-270).
+            for (int t = lane; t < n; t += 64)
             {
-                int const ak = A.nbrJ[o + k];
-                int const ek = A.elem[ak];
-                if (!weighted
-                    && !((g.e1 == ej && g.e2 == ek) || (g.e2 == ej && g.e1 == ek)))
-                    continue;
-                double4 const gk = A.geo[o + k];
-                double const rik = gk.w;
-                if (!(rik < g.rc)) continue;
-                double const jx = gk.x - gj.x, jy = gk.y - gj.y,
-                             jz = gk.z - gj.z;
-                double rjk = jx * jx + jy * jy + jz * jz;
-                if (!wide && !(rjk < g.rc2)) continue;
-                rjk = sqrt(rjk);
-                double fcik, dfcik, fcjk = 1.0, dfcjk = 0.0;
-                cutoff_fdf<double>(cc, rik, fcik, dfcik);
-                if (!wide) cutoff_fdf<double>(cc, rjk, fcjk, dfcjk);
-                double const dk0 = A.F[3 * (size_t)ak] - A.Fref[3 * (size_t)ak];
-                double const dk1 = A.F[3 * (size_t)ak + 1]
-                                 - A.Fref[3 * (size_t)ak + 1];
-                double const dk2 = A.F[3 * (size_t)ak + 2]
-                                 - A.Fref[3 * (size_t)ak + 2];
-                double const tij = (gj.x * (da[0] - dj[0]) + gj.y * (da[1] - dj[1])
-                                    + gj.z * (da[2] - dj[2]));
-                double const tik = (gk.x * (da[0] - dk0) + gk.y * (da[1] - dk1)
-                                    + gk.z * (da[2] - dk2));
-                double const tjk = (jx * (dk0 - dj[0]) + jy * (dk1 - dj[1])
-                                    + jz * (dk2 - dj[2]));
-                double const rinv = 1.0 / rij / rik;
-                double const cost = (gj.x * gk.x + gj.y * gk.y + gj.z * gk.z)
-                                  * rinv;
-                // Weighted type 13: the cutoff products times Z_j Z_k
-                // (SymGrpExpAngnWeighted.cpp:263-270).
-                double const z = weighted ? T.zw[ej] * T.zw[ek] : 1.0;
-                double const pfc = z * fcij * fcik * fcjk;
+                double f, df;
+                cutoff_fdf_t<CT>(cc, P[t].w, f, df);
+                if (weighted)
+                {
+                    double const z = staged_weight(T, sStart, sCnt, t);
+                    f *= z;
+                    df *= z;
+                }
+                Q[t].x = f;
+                Q[t].z = df * Q[t].y;
+            }
+            keyCached = key;
+        }
+        __syncthreads();
+        double acc[MAXM];
 #pragma unroll
-                for (int q = 0; q < kMaxMembers; ++q)
-                    if (q < g.nmem)
+        for (int m = 0; m < MAXM; ++m) acc[m] = 0.0;
+        if (sf_radial(g.type))
+        {
+            int const a0 = weighted ? 0 : sStart[g.e1];
+            int const na = weighted ? n : sCnt[g.e1];
+            for (int t = lane; t < na; t += 64)
+            {
+                double const r = P[a0 + t].w;
+                if (!(r < g.rc)) continue;
+                double4 const q = Q[a0 + t];
+                double const df = q.z * q.w, f2 = 2.0 * q.x * (q.y * q.w);
+#pragma unroll
+                for (int m = 0; m < MAXM; ++m)
+                    if (m < nmem)
                     {
-                        MemberDesc const& md = mem[q];
-                        double const rijs = rij - md.rs, riks = rik - md.rs,
-                                     rjks = rjk - md.rs;
-                        double const ex = wide
-                            ? exp(-md.eta * (rijs * rijs + riks * riks))
-                            : exp(-md.eta * (rijs * rijs + riks * riks
-                                             + rjks * rjks));
-                        double const pl = 1.0 + md.lambda * cost;
-                        if (pl <= 0.0) continue;
-                        double fg = ex * (md.useint ? pow_int(pl, md.zint - 1)
-                                                    : pow(pl, md.zeta - 1.0));
-                        fg *= pow(2.0, 1.0 - md.zeta);
-                        double const pzl = md.zeta * md.lambda;
-                        double const ri = rinv * pzl, ct = cost * pzl;
-                        double const p2e = 2.0 * md.eta * pl;
-                        double const p1 = fg * (pfc * (ri - ct / (rij * rij)
-                                                - p2e * rijs / rij)
-                                                + z * fcik * fcjk * dfcij * pl
-                                                / rij);
-                        double const p2 = fg * (pfc * (ri - ct / (rik * rik)
-                                                - p2e * riks / rik)
-                                                + z * fcij * fcjk * dfcik * pl
-                                                / rik);
-                        double const p3 = wide
-                            ? fg * pfc * ri
-                            : fg * (pfc * (ri + p2e * rjks / rjk)
-                                    - z * fcij * fcik * dfcjk * pl / rjk);
-                        acc[q] += md.sfac * (p1 * tij + p2 * tik + p3 * tjk);
+                        double const eta = MP[m].eta, x = r - MP[m].rs;
+                        acc[m] += (df - eta * x * f2) * exp(-eta * x * x);
                     }
             }
         }
+        else
+        {
+            bool const wide = g.type == 9;
+            DiagPairs const dp = weighted
+                ? DiagPairs(true, 0, n, 0, n)
+                : DiagPairs(g.e1 == g.e2, sStart[g.e1], sCnt[g.e1],
+                            sStart[g.e2], sCnt[g.e2]);
+            double lam[MAXM], zl[MAXM];
+            int code[MAXM];
 #pragma unroll
-        for (int q = 0; q < kMaxMembers; ++q)
-            if (q < g.nmem)
+            for (int m = 0; m < MAXM; ++m)
             {
-                double const s = wave_sum(acc[q]);
-                if (lane == 0) U[mem[q].sf] = A.cF * s;
+                MParam<double> const& p = MP[m < nmem ? m : 0];
+                lam[m] = uniform_r(p.lambda);
+                zl[m] = uniform_r(p.zl);
+                code[m] = uniform(p.flags);
             }
+            auto triplet = [&](int j, int k) {
+                double4 const pj = P[j], pk = P[k], qj = Q[j], qk = Q[k];
+                double const dx = pk.x - pj.x, dy = pk.y - pj.y,
+                             dz = pk.z - pj.z;
+                double const tjk = dx * (E[j] - E[k])
+                                 + dy * (E[cap + j] - E[cap + k])
+                                 + dz * (E[2 * cap + j] - E[2 * cap + k]);
+                double const rinv = qj.y * qk.y;
+                double const cost = (pj.x * pk.x + pj.y * pk.y + pj.z * pk.z)
+                                  * rinv;
+                double const fij_ik = qj.x * qk.x;
+                double pfc = fij_ik, r2sum = pj.w * pj.w + pk.w * pk.w;
+                double B = qk.x * qj.z * qj.w + qj.x * qk.z * qk.w;
+                double C = qj.w + qk.w, rjk = 0.0, injk = 0.0;
+                if (!wide)
+                {
+                    double const rjk2 = dx * dx + dy * dy + dz * dz;
+                    injk = rsqrt_nr(rjk2);
+                    rjk = rjk2 * injk;
+                    double fcjk, dfcjk;
+                    cutoff_inside<CT>(cc, rjk, fcjk, dfcjk);
+                    pfc *= fcjk;
+                    r2sum += rjk2;
+                    B = B * fcjk - fij_ik * (dfcjk * injk) * tjk;
+                    C -= tjk;
+                }
+                double const Av = pfc * (rinv * (qj.w + qk.w + tjk)
+                                         - cost * (qj.w * (qj.y * qj.y)
+                                                   + qk.w * (qk.y * qk.y)));
+                double ex = 0.0, BC = 0.0, pl = 0.0;
+                PowChain<double> chain;
+                chain.reset(0.0);
+#pragma unroll
+                for (int m = 0; m < MAXM; ++m)
+                    if (m < nmem)
+                    {
+                        int const fl = code[m];
+                        if (fl & MF_NEWEXP)
+                        {
+                            double const eta = MP[m].eta, rs = MP[m].rs;
+                            double s = r2sum, c = C;
+                            if (rs != 0.0)
+                            {
+                                double const x = pj.w - rs, y = pk.w - rs;
+                                s = x * x + y * y;
+                                c = x * qj.y * qj.w + y * qk.y * qk.w;
+                                if (!wide)
+                                {
+                                    double const w = rjk - rs;
+                                    s += w * w;
+                                    c -= w * injk * tjk;
+                                }
+                            }
+                            ex = exp(-eta * s);
+                            BC = B - 2.0 * eta * pfc * c;
+                        }
+                        if (fl & MF_NEWLAM)
+                        {
+                            pl = 1.0 + lam[m] * cost;
+                            chain.reset(pl);
+                        }
+                        double pw;
+                        if (fl & MF_PREFIX) pw = chain.at((fl >> 8) & 15);
+                        else if (!GENPOW || (fl & MF_INTPOW))
+                            pw = pow_int(pl, MP[m].zint - 1);
+                        else pw = pow(pl, MP[m].zeta - 1.0);
+                        acc[m] += pl > 0.0 ? ex * pw * (zl[m] * Av + pl * BC)
+                                           : 0.0;
+                    }
+            };
+            int qn = 0, pc = 0, pr = 0;
+            dp.start(lane, pc, pr);
+            for (int base = 0; base < dp.npairs; base += 64)
+            {
+                bool const valid = base + lane < dp.npairs;
+                int j, k;
+                dp.pair(pc, pr, j, k);
+                if (!valid) j = k = dp.s0;
+                dp.advance(pc, pr);
+                bool const pass = valid
+                    & pair_in_range<double>(P[j], P[k], wide, g.rc, g.rc2);
+                uint64_t const mask = __ballot(pass);
+                if (pass) QUEUE[qn + lanes_below(mask)] = j | (k << 16);
+                qn += __popcll(mask);
+                wave_lds_fence();
+                if (qn >= 64)
+                {
+                    int const e = QUEUE[qn - 64 + lane];
+                    triplet(e & 0xffff, e >> 16);
+                    qn -= 64;
+                    wave_lds_fence();
+                }
+            }
+            if (lane < qn)
+            {
+                int const e = QUEUE[lane];
+                triplet(e & 0xffff, e >> 16);
+            }
+        }
+        // Member m's total ends in the lanes (m << kSh) + t.
+        double const v = wave_sum_transposed<MAXM>(acc);
+        constexpr int kSh = MAXM == 8 ? 3 : 2;   // 6 - log2 MAXM
+        int const m = lane >> kSh;
+        if ((lane & ((1 << kSh) - 1)) == 0 && m < nmem)
+        {
+            MemberDesc const& md = mem[m];
+            U[md.sf] = A.cF * v * (sf_radial(g.type)
+                                   ? scale_slope(T.scale[ed.sf0 + md.sf])
+                                   : md.fnorm);
+        }
+        __syncthreads();
     }
+}
+
+template <int MAXM>
+void launch_train_u_m(TrainArgs const& A, hipStream_t s)
+{
+    size_t const shm = force_backward_lds_bytes(A.cap, 0);
+    if (A.T.genpow)
+        HDNNP_CUTOFF_DISPATCH(A.T.cutType,
+            (k_train_u<MAXM, kCT, true><<<A.n, 64, shm, s>>>(A)));
+    else
+        HDNNP_CUTOFF_DISPATCH(A.T.cutType,
+            (k_train_u<MAXM, kCT, false><<<A.n, 64, shm, s>>>(A)));
 }
 
 // Per-block gradient of sum over the block's atoms of
@@ -698,7 +825,10 @@ size_t train_lds_per_atom(ElemDesc const& ed)
 hipError_t launch_train_u(TrainArgs const& A, hipStream_t s)
 {
     if (A.n <= 0) return hipSuccess;
-    k_train_u<<<A.n, 64, 0, s>>>(A);
+    // The LDS of the FP64 force kernel, which ran before on the same list:
+    // 11 doubles per staged neighbour and the pair queue.
+    if (A.T.maxGroupMembers <= 8) launch_train_u_m<8>(A, s);
+    else launch_train_u_m<kMaxMembers>(A, s);
     return hipGetLastError();
 }
 
