@@ -2642,19 +2642,19 @@ int hdnnp_train_gradient(hdnnp_ctx* c, const double* f_ref, double e_ref,
                             "compact training kernel's LDS staging.\n");
             hipCheck(launch_train_u_compact(A, cap, s), "train u (compact)");
         }
-        for (size_t e = 0; e < c->flat.elem.size(); ++e)
         {
-            ElemDesc const& ed = c->flat.elem[e];
-            int const per = train_atoms_per_grad_block(ed);
-            int nwe = 0;
-            for (int l = 1; l < ed.nlayers; ++l)
-                nwe += ed.width[l] * ed.width[l - 1] + ed.width[l];
-            int const na = (int)c->hAtomsOfElem[e].size();
-            int const nb = (na + per - 1) / per;
-            c->tPart.ensure((size_t)std::max(nb, 1) * nwe);
-            hipCheck(launch_train_grad(A, ed, (int)e, c->dAtomsOfElem[e].p, na,
-                                       c->tPart.p, nwe,
-                                       c->tGrad.p + ed.woff[1], s),
+            int const* atoms[kMaxElements] = {};
+            int na[kMaxElements] = {};
+            size_t np = 0;
+            for (int e = 0; e < c->T.ne; ++e)
+            {
+                atoms[e] = c->dAtomsOfElem[e].p;
+                na[e] = (int)c->hAtomsOfElem[e].size();
+                np += train_grad_partials(c->flat.elem[e], na[e]);
+            }
+            c->tPart.ensure(std::max<size_t>(np, 1));
+            hipCheck(launch_train_grad(A, c->flat.elem.data(), atoms, na,
+                                       c->tPart.p, c->tGrad.p, s),
                      "train gradient");
         }
         hipCheck(launch_energy_sum(c->tD2.p, n, c->tLoss.p, s), "train loss");

@@ -108,9 +108,13 @@ hipError_t launch_train_u(TrainArgs const& A, hipStream_t s);
 // neighbour count.
 hipError_t launch_train_u_compact(TrainArgs const& A, int cap, hipStream_t s);
 size_t train_u_compact_lds_bytes(ModelTables const& T, int cap);
-hipError_t launch_train_grad(TrainArgs const& A, ElemDesc const& ed, int e,
-                             const int* atoms, int na, double* part, int nw,
-                             double* grad, hipStream_t s);
+// The loss gradient of all elements' weights in one launch: per element e its
+// atoms and their number, part with room for the sum over the elements of
+// train_grad_partials doubles, grad in the flat weight order.
+size_t train_grad_partials(ElemDesc const& ed, int na);
+hipError_t launch_train_grad(TrainArgs const& A, ElemDesc const* eds,
+                             const int* const* atoms, const int* na,
+                             double* part, double* grad, hipStream_t s);
 hipError_t launch_adam(int n, double* w, float* w32, const double* g,
                        double* m, double* v, double lr, double b1, double b2,
                        double eps, int64_t step, hipStream_t s);

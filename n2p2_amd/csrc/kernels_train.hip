@@ -28,6 +28,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <climits>
 #include <cmath>
 
 #include "device_common.h"
@@ -376,26 +377,49 @@ void launch_train_u_m(TrainArgs const& A, hipStream_t s)
 }
 
 // Per-block gradient of sum over the block's atoms of
-// kappa E_a + (derivative of E_a along u_a), atoms of element e, apb per
+// kappa E_a + (derivative of E_a along u_a), apb atoms of one element per
 // block.  LDS per atom: the inputs x, tangents t of every layer and the
 // adjoints of z and s of every layer, plus two adjoint scratch vectors.
+//
+// The threads of the block share every layer: thread t takes atom t % apb and
+// every (256 / apb)-th neuron, so a wave reads one or two weight rows
+// (broadcast) and the atoms' LDS records at an odd stride (no bank
+// conflicts).  Each neuron's sum still runs over its inputs in order.  With
+// one thread per atom, as before, the serial chain of the whole network
+// bounded the kernel (200 us per element whatever the size of the
+// structure); the elements now also run in one launch: 404 -> 33 us for both
+// elements of a 1,536-atom water box (40-25-25-1).
 constexpr int kAtoms = 32;
+constexpr int kGradThreads = 256;
 
-__global__ __launch_bounds__(64) void k_train_grad(TrainArgs A, int e,
-                                                   const int* __restrict__ atoms,
-                                                   int na, int perAtom,
-                                                   int apb,
-                                                   double* __restrict__ part,
-                                                   int nw)
+// One launch covers all elements (blockIdx.y).
+struct TrainGradTab
+{
+    const int* atoms[kMaxElements];
+    int na[kMaxElements], nb[kMaxElements], nw[kMaxElements];
+    int stride[kMaxElements], apb[kMaxElements];
+    size_t off[kMaxElements];    // the element's offset in the partials
+};
+
+__global__ __launch_bounds__(kGradThreads) void k_train_grad(
+    TrainArgs A, TrainGradTab G, double* __restrict__ partAll)
 {
     extern __shared__ double lds[];
+    int const e = blockIdx.y, b = blockIdx.x;
+    if (b >= G.nb[e]) return;
     ModelTables const& T = A.T;
     ElemDesc const& ed = T.elem[e];
     int const L = ed.nlayers - 1;
     int const t = threadIdx.x;
-    int const b = blockIdx.x;
-    int const nat = min(apb, na - b * apb);
+    int const apb = G.apb[e], perAtom = G.stride[e], nw = G.nw[e];
+    int const nat = min(apb, G.na[e] - b * apb);
+    int const* __restrict__ atoms = G.atoms[e] + b * apb;
     const double* __restrict__ W = T.weights;
+    // Thread -> (atom q, first neuron k0, neuron step).
+    int const kstep = kGradThreads / apb;
+    int const q = t % apb;
+    int const k0 = q < nat && t / apb < kstep ? t / apb : INT_MAX / 2;
+    double* const P = lds + (size_t)q * perAtom;
     // LDS layout per atom: for l = 1..L: X[l-1] (w_{l-1}), Tg[l-1]
     // (w_{l-1}), Z[l] (w_l), S[l] (w_l); then Xb, Tb (maxwidth each).
     int lo[kMaxLayers];   // offset of layer l's block within an atom
@@ -410,90 +434,95 @@ __global__ __launch_bounds__(64) void k_train_grad(TrainArgs A, int e,
     }
     double const kappa = 2.0 * A.wE * (A.energy[0] - A.Eref)
                        / ((double)A.n * (double)A.n);
-    if (t < nat)
+    // inputs: scaled G and its tangent u
     {
-        int const a = atoms[b * apb + t];
-        double* __restrict__ P = lds + (size_t)t * perAtom;
-        // inputs: scaled G and its tangent u
+        int const w0 = ed.width[0];
+        for (int idx = t; idx < nat * w0; idx += kGradThreads)
         {
-            double* X0 = P + lo[1];
-            double* T0 = X0 + ed.width[0];
-            for (int j = 0; j < ed.width[0]; ++j)
-            {
-                X0[j] = A.G[(size_t)a * A.ldG + j];
-                T0[j] = A.U[(size_t)a * A.ldG + j];
-            }
-        }
-        // forward with tangent
-        for (int l = 1; l <= L; ++l)
-        {
-            int const nin = ed.width[l - 1], nout = ed.width[l];
-            double* X = P + lo[l];
-            double* Tg = X + nin;
-            double* Z = Tg + nin;
-            double* S = Z + nout;
-            double* Xn = l < L ? P + lo[l + 1] : nullptr;
-            double* Tn = l < L ? Xn + nout : nullptr;
-            const double* Wl = W + ed.woff[l];
-            const double* bl = W + ed.boff[l];
-            for (int k = 0; k < nout; ++k)
-            {
-                double z = bl[k], s = 0.0;
-                for (int j = 0; j < nin; ++j)
-                {
-                    z += Wl[(size_t)k * nin + j] * X[j];
-                    s += Wl[(size_t)k * nin + j] * Tg[j];
-                }
-                Z[k] = z;
-                S[k] = s;
-                if (l < L)
-                {
-                    double v, d, dd;
-                    activate2(ed.act[l], z, v, d, dd);
-                    Xn[k] = v;
-                    Tn[k] = d * s;
-                }
-            }
-        }
-        // reverse through value and tangent
-        double* Xb = P + lo[0];
-        double* Tb = Xb + ed.maxwidth;
-        Xb[0] = kappa;
-        Tb[0] = 1.0;
-        for (int l = L; l >= 1; --l)
-        {
-            int const nin = ed.width[l - 1], nout = ed.width[l];
-            double* X = P + lo[l];
-            double* Z = X + 2 * nin;
-            double* S = Z + nout;
-            const double* Wl = W + ed.woff[l];
-            for (int k = 0; k < nout; ++k)
-            {
-                double v, d, dd;
-                activate2(ed.act[l], Z[k], v, d, dd);
-                double const zb = Xb[k] * d + Tb[k] * S[k] * dd;
-                double const sb = Tb[k] * d;
-                Z[k] = zb;       // adjoint of z replaces z
-                S[k] = sb;       // adjoint of s replaces s
-            }
-            if (l > 1)
-                for (int j = 0; j < nin; ++j)
-                {
-                    double xb = 0.0, tb = 0.0;
-                    for (int k = 0; k < nout; ++k)
-                    {
-                        xb += Wl[(size_t)k * nin + j] * Z[k];
-                        tb += Wl[(size_t)k * nin + j] * S[k];
-                    }
-                    Xb[j] = xb;
-                    Tb[j] = tb;
-                }
+            int const m = idx / w0, j = idx - m * w0;
+            size_t const g = (size_t)atoms[m] * A.ldG + j;
+            double* X0 = lds + (size_t)m * perAtom + lo[1];
+            X0[j] = A.G[g];
+            X0[w0 + j] = A.U[g];
         }
     }
     __syncthreads();
+    // forward with tangent
+    for (int l = 1; l <= L; ++l)
+    {
+        int const nin = ed.width[l - 1], nout = ed.width[l];
+        double const* X = P + lo[l];
+        double const* Tg = X + nin;
+        double* Z = P + lo[l] + 2 * nin;
+        double* Xn = l < L ? P + lo[l + 1] : nullptr;
+        for (int k = k0; k < nout; k += kstep)
+        {
+            double const* Wk = W + ed.woff[l] + (size_t)k * nin;
+            double z = W[ed.boff[l] + k], s = 0.0;
+#pragma unroll 4
+            for (int j = 0; j < nin; ++j)
+            {
+                z += Wk[j] * X[j];
+                s += Wk[j] * Tg[j];
+            }
+            Z[k] = z;
+            Z[nout + k] = s;
+            if (l < L)
+            {
+                double v, d, dd;
+                activate2(ed.act[l], z, v, d, dd);
+                Xn[k] = v;
+                Xn[nout + k] = d * s;
+            }
+        }
+        __syncthreads();
+    }
+    // reverse through value and tangent
+    double* Xb = P + lo[0];
+    double* Tb = Xb + ed.maxwidth;
+    if (k0 == 0)
+    {
+        Xb[0] = kappa;
+        Tb[0] = 1.0;
+    }
+    __syncthreads();
+    for (int l = L; l >= 1; --l)
+    {
+        int const nin = ed.width[l - 1], nout = ed.width[l];
+        double* Z = P + lo[l] + 2 * nin;
+        double* S = Z + nout;
+        double const* Wl = W + ed.woff[l];
+        for (int k = k0; k < nout; k += kstep)
+        {
+            double v, d, dd;
+            activate2(ed.act[l], Z[k], v, d, dd);
+            double const zb = Xb[k] * d + Tb[k] * S[k] * dd;
+            double const sb = Tb[k] * d;
+            Z[k] = zb;       // adjoint of z replaces z
+            S[k] = sb;       // adjoint of s replaces s
+        }
+        __syncthreads();
+        if (l > 1)
+        {
+            for (int j = k0; j < nin; j += kstep)
+            {
+                double xb = 0.0, tb = 0.0;
+#pragma unroll 4
+                for (int k = 0; k < nout; ++k)
+                {
+                    xb += Wl[(size_t)k * nin + j] * Z[k];
+                    tb += Wl[(size_t)k * nin + j] * S[k];
+                }
+                Xb[j] = xb;
+                Tb[j] = tb;
+            }
+            __syncthreads();
+        }
+    }
     // dW_l[k][j] = sum_atoms zb_k x_j + sb_k t_j;  db_l[k] = sum_atoms zb_k
+    double* __restrict__ part = partAll + G.off[e] + (size_t)b * nw;
     int const base = ed.woff[1];
-    for (int idx = t; idx < nw; idx += 64)
+    for (int idx = t; idx < nw; idx += kGradThreads)
     {
         int const gidx = base + idx;
         int l = 1;
@@ -504,9 +533,9 @@ __global__ __launch_bounds__(64) void k_train_grad(TrainArgs A, int e,
         {
             int const r = gidx - ed.woff[l];
             int const k = r / nin, j = r - k * nin;
-            for (int q = 0; q < nat; ++q)
+            for (int m = 0; m < nat; ++m)
             {
-                double const* X = lds + (size_t)q * perAtom + lo[l];
+                double const* X = lds + (size_t)m * perAtom + lo[l];
                 double const* Z = X + 2 * nin;
                 acc += Z[k] * X[j] + Z[nout + k] * X[nin + j];
             }
@@ -514,22 +543,27 @@ __global__ __launch_bounds__(64) void k_train_grad(TrainArgs A, int e,
         else
         {
             int const k = gidx - ed.boff[l];
-            for (int q = 0; q < nat; ++q)
-                acc += (lds + (size_t)q * perAtom + lo[l])[2 * nin + k];
+            for (int m = 0; m < nat; ++m)
+                acc += (lds + (size_t)m * perAtom + lo[l])[2 * nin + k];
         }
-        part[(size_t)b * nw + idx] = acc;
+        part[idx] = acc;
     }
 }
 
-// grad[base + idx] = sum over blocks of part (fixed order).
-__global__ void k_train_reduce(const double* __restrict__ part, int nb,
-                               int nw, double* __restrict__ grad)
+// grad[base + idx] = sum over the element's blocks of part (fixed order).
+__global__ void k_train_reduce(TrainGradTab G, ModelTables T,
+                               const double* __restrict__ partAll,
+                               double* __restrict__ grad)
 {
+    int const e = blockIdx.y;
     int const idx = blockIdx.x * blockDim.x + threadIdx.x;
+    int const nw = G.nw[e];
     if (idx >= nw) return;
+    const double* __restrict__ part = partAll + G.off[e];
     double acc = 0.0;
-    for (int b = 0; b < nb; ++b) acc += part[(size_t)b * nw + idx];
-    grad[idx] = acc;
+#pragma unroll 8
+    for (int b = 0; b < G.nb[e]; ++b) acc += part[(size_t)b * nw + idx];
+    grad[T.elem[e].woff[1] + idx] = acc;
 }
 
 // Adam (Kingma & Ba 2015, Algorithm 1) on w with gradient g at step t >= 1.
@@ -563,8 +597,9 @@ __global__ void k_to_f32(int n, const double* __restrict__ w,
 // atom's network (NeuralNetwork::calculateDEdc, NeuralNetwork.cpp:444-490),
 // then per weight the sum over the block's atoms in atom order.  LDS per
 // atom: for every layer its input x and the adjoint of z, plus one adjoint
-// scratch vector.
-__global__ __launch_bounds__(64) void k_energy_wgrad(
+// scratch vector.  Threads share the layers as in k_train_grad (one thread
+// per atom took 230 us for a 192-atom structure, now 39 us).
+__global__ __launch_bounds__(kGradThreads) void k_energy_wgrad(
     ModelTables T, const double* __restrict__ G, int ldG,
     const int* __restrict__ blkAtoms, const int* __restrict__ blk0,
     const int* __restrict__ blkN, const int* __restrict__ blkElem,
@@ -577,7 +612,12 @@ __global__ __launch_bounds__(64) void k_energy_wgrad(
     ElemDesc const& ed = T.elem[e];
     int const L = ed.nlayers - 1;
     int const nat = blkN[b];
+    int const* __restrict__ atoms = blkAtoms + blk0[b];
     const double* __restrict__ W = T.weights;
+    constexpr int kstep = kGradThreads / kAtoms;
+    int const q = t % kAtoms;
+    int const k0 = q < nat ? t / kAtoms : INT_MAX / 2;
+    double* const P = lds + (size_t)q * perAtom;
     int lo[kMaxLayers];
     {
         int p = 0;
@@ -588,63 +628,70 @@ __global__ __launch_bounds__(64) void k_energy_wgrad(
         }
         lo[0] = p;
     }
-    if (t < nat)
     {
-        int const a = blkAtoms[blk0[b] + t];
-        double* __restrict__ P = lds + (size_t)t * perAtom;
-        for (int j = 0; j < ed.width[0]; ++j)
-            P[lo[1] + j] = G[(size_t)a * ldG + j];
-        for (int l = 1; l <= L; ++l)
+        int const w0 = ed.width[0];
+        for (int idx = t; idx < nat * w0; idx += kGradThreads)
         {
-            int const nin = ed.width[l - 1], nout = ed.width[l];
-            double* X = P + lo[l];
-            double* Z = X + nin;
-            double* Xn = l < L ? P + lo[l + 1] : nullptr;
-            const double* Wl = W + ed.woff[l];
-            const double* bl = W + ed.boff[l];
-            for (int k = 0; k < nout; ++k)
-            {
-                double z = bl[k];
-                for (int j = 0; j < nin; ++j)
-                    z += Wl[(size_t)k * nin + j] * X[j];
-                Z[k] = z;
-                if (l < L)
-                {
-                    double v, d;
-                    activate(ed.act[l], z, v, d);
-                    Xn[k] = v;
-                }
-            }
-        }
-        double* Xb = P + lo[0];
-        for (int k = 0; k < ed.width[L]; ++k) Xb[k] = 1.0;
-        for (int l = L; l >= 1; --l)
-        {
-            int const nin = ed.width[l - 1], nout = ed.width[l];
-            double* X = P + lo[l];
-            double* Z = X + nin;
-            const double* Wl = W + ed.woff[l];
-            for (int k = 0; k < nout; ++k)
-            {
-                double v, d;
-                activate(ed.act[l], Z[k], v, d);
-                Z[k] = Xb[k] * d;        // adjoint of z replaces z
-            }
-            if (l > 1)
-                for (int j = 0; j < nin; ++j)
-                {
-                    double xb = 0.0;
-                    for (int k = 0; k < nout; ++k)
-                        xb += Wl[(size_t)k * nin + j] * Z[k];
-                    Xb[j] = xb;
-                }
+            int const m = idx / w0, j = idx - m * w0;
+            (lds + (size_t)m * perAtom + lo[1])[j]
+                = G[(size_t)atoms[m] * ldG + j];
         }
     }
     __syncthreads();
+    for (int l = 1; l <= L; ++l)
+    {
+        int const nin = ed.width[l - 1], nout = ed.width[l];
+        double const* X = P + lo[l];
+        double* Z = P + lo[l] + nin;
+        double* Xn = l < L ? P + lo[l + 1] : nullptr;
+        for (int k = k0; k < nout; k += kstep)
+        {
+            double const* Wk = W + ed.woff[l] + (size_t)k * nin;
+            double z = W[ed.boff[l] + k];
+#pragma unroll 4
+            for (int j = 0; j < nin; ++j) z += Wk[j] * X[j];
+            Z[k] = z;
+            if (l < L)
+            {
+                double v, d;
+                activate(ed.act[l], z, v, d);
+                Xn[k] = v;
+            }
+        }
+        __syncthreads();
+    }
+    double* Xb = P + lo[0];
+    for (int k = k0; k < ed.width[L]; k += kstep) Xb[k] = 1.0;
+    __syncthreads();
+    for (int l = L; l >= 1; --l)
+    {
+        int const nin = ed.width[l - 1], nout = ed.width[l];
+        double* Z = P + lo[l] + nin;
+        const double* Wl = W + ed.woff[l];
+        for (int k = k0; k < nout; k += kstep)
+        {
+            double v, d;
+            activate(ed.act[l], Z[k], v, d);
+            Z[k] = Xb[k] * d;        // adjoint of z replaces z
+        }
+        __syncthreads();
+        if (l > 1)
+        {
+            for (int j = k0; j < nin; j += kstep)
+            {
+                double xb = 0.0;
+#pragma unroll 4
+                for (int k = 0; k < nout; ++k)
+                    xb += Wl[(size_t)k * nin + j] * Z[k];
+                Xb[j] = xb;
+            }
+            __syncthreads();
+        }
+    }
     int const base = ed.woff[1];
     int nw = 0;
     for (int l = 1; l <= L; ++l) nw += ed.width[l] * ed.width[l - 1] + ed.width[l];
-    for (int idx = t; idx < nw; idx += 64)
+    for (int idx = t; idx < nw; idx += kGradThreads)
     {
         int const gidx = base + idx;
         int l = 1;
@@ -655,40 +702,39 @@ __global__ __launch_bounds__(64) void k_energy_wgrad(
         {
             int const r = gidx - ed.woff[l];
             int const k = r / nin, j = r - k * nin;
-            for (int q = 0; q < nat; ++q)
+            for (int m = 0; m < nat; ++m)
             {
-                double const* X = lds + (size_t)q * perAtom + lo[l];
+                double const* X = lds + (size_t)m * perAtom + lo[l];
                 acc += X[nin + k] * X[j];
             }
         }
         else
         {
             int const k = gidx - ed.boff[l];
-            for (int q = 0; q < nat; ++q)
-                acc += (lds + (size_t)q * perAtom + lo[l])[nin + k];
+            for (int m = 0; m < nat; ++m)
+                acc += (lds + (size_t)m * perAtom + lo[l])[nin + k];
         }
         part[(size_t)b * maxP + idx] = acc;
     }
 }
 
 // J[s][base_e + idx] = sum over the blocks of (structure s, element e), in
-// block order.  One workgroup per (s, e); blocks of (s, e) are
-// [grp0[s*ne+e], grp0[s*ne+e+1]).
-__global__ void k_energy_wgrad_reduce(const double* __restrict__ part,
-                                      int maxP, const int* __restrict__ grp0,
-                                      const int* __restrict__ base,
-                                      const int* __restrict__ nwe, int ne,
-                                      int nwTotal, double* __restrict__ J)
+// block order.  One workgroup per (s, e) and 256 weights; blocks of (s, e)
+// are [grp0[s*ne+e], grp0[s*ne+e+1]).
+__global__ __launch_bounds__(256) void k_energy_wgrad_reduce(
+    const double* __restrict__ part, int maxP, const int* __restrict__ grp0,
+    const int* __restrict__ base, const int* __restrict__ nwe, int ne,
+    int nwTotal, double* __restrict__ J)
 {
     int const se = blockIdx.x;
     int const s = se / ne, e = se - s * ne;
     int const b0 = grp0[se], b1 = grp0[se + 1];
-    for (int idx = threadIdx.x; idx < nwe[e]; idx += blockDim.x)
-    {
-        double acc = 0.0;
-        for (int b = b0; b < b1; ++b) acc += part[(size_t)b * maxP + idx];
-        J[(size_t)s * nwTotal + base[e] + idx] = acc;
-    }
+    int const idx = blockIdx.y * 256 + threadIdx.x;
+    if (idx >= nwe[e]) return;
+    double acc = 0.0;
+#pragma unroll 4
+    for (int b = b0; b < b1; ++b) acc += part[(size_t)b * maxP + idx];
+    J[(size_t)s * nwTotal + base[e] + idx] = acc;
 }
 
 // Kalman filter, one scalar observation (KalmanFilter.cpp:126-196 with
@@ -793,25 +839,42 @@ hipError_t launch_energy_wgrad(ModelTables const& T, const double* G, int ldG,
                                const int* nwe, int ne, int nstruct,
                                int nwTotal, double* J, hipStream_t s)
 {
+    // An odd record stride where it fits (the caller checked perAtom).
+    int const odd = perAtom | 1;
+    int const stride = (size_t)odd * kAtoms * sizeof(double) <= 65536
+                     ? odd : perAtom;
     if (nblk > 0)
-        k_energy_wgrad<<<nblk, 64, (size_t)perAtom * kAtoms * sizeof(double),
-                         s>>>(T, G, ldG, blkAtoms, blk0, blkN, blkElem,
-                              perAtom, part, maxP);
+        k_energy_wgrad<<<nblk, kGradThreads,
+                         (size_t)stride * kAtoms * sizeof(double), s>>>(
+            T, G, ldG, blkAtoms, blk0, blkN, blkElem, stride, part, maxP);
     if (nstruct * ne > 0)
-        k_energy_wgrad_reduce<<<nstruct * ne, 256, 0, s>>>(
-            part, maxP, grp0, base, nwe, ne, nwTotal, J);
+        k_energy_wgrad_reduce<<<dim3(nstruct * ne, (maxP + 255) / 256), 256,
+                                0, s>>>(part, maxP, grp0, base, nwe, ne,
+                                        nwTotal, J);
     return hipGetLastError();
 }
 
 int train_atoms_per_block() { return kAtoms; }
+
+namespace {
+
+// Doubles between the atoms' LDS records of the loss-gradient kernel: odd
+// unless only the exact size fits.
+size_t train_lds_stride(ElemDesc const& ed)
+{
+    size_t const per = train_lds_per_atom(ed);
+    return (per | 1) * sizeof(double) <= 65536 ? per | 1 : per;
+}
+
+}  // namespace
 
 // Atoms per block of the loss-gradient kernel: up to kAtoms, fewer for wide
 // networks so that their LDS stays within 64 KiB (0 if one atom does not
 // fit).
 int train_atoms_per_grad_block(ElemDesc const& ed)
 {
-    size_t const per = train_lds_per_atom(ed) * sizeof(double);
-    return (int)std::min<size_t>(kAtoms, 65536 / per);
+    return (int)std::min<size_t>(kAtoms, 65536 / (train_lds_stride(ed)
+                                                  * sizeof(double)));
 }
 
 size_t train_lds_per_atom(ElemDesc const& ed)
@@ -832,21 +895,44 @@ hipError_t launch_train_u(TrainArgs const& A, hipStream_t s)
     return hipGetLastError();
 }
 
-hipError_t launch_train_grad(TrainArgs const& A, ElemDesc const& ed, int e,
-                             const int* atoms, int na, double* part, int nw,
-                             double* grad, hipStream_t s)
+size_t train_grad_partials(ElemDesc const& ed, int na)
 {
-    if (na <= 0)
+    size_t const apb = std::max(train_atoms_per_grad_block(ed), 1);
+    size_t nw = 0;
+    for (int l = 1; l < ed.nlayers; ++l)
+        nw += (size_t)ed.width[l] * ed.width[l - 1] + ed.width[l];
+    return nw * ((na + apb - 1) / apb);
+}
+
+hipError_t launch_train_grad(TrainArgs const& A, ElemDesc const* eds,
+                             const int* const* atoms, const int* na,
+                             double* part, double* grad, hipStream_t s)
+{
+    TrainGradTab G{};
+    size_t off = 0, shm = 0;
+    int nb = 0, nw = 0;
+    for (int e = 0; e < A.T.ne; ++e)
     {
-        k_train_reduce<<<(nw + 255) / 256, 256, 0, s>>>(part, 0, nw, grad);
-        return hipGetLastError();
+        ElemDesc const& ed = eds[e];
+        G.atoms[e] = atoms[e];
+        G.na[e] = na[e];
+        G.apb[e] = train_atoms_per_grad_block(ed);
+        G.stride[e] = (int)train_lds_stride(ed);
+        G.nb[e] = (na[e] + G.apb[e] - 1) / G.apb[e];
+        for (int l = 1; l < ed.nlayers; ++l)
+            G.nw[e] += ed.width[l] * ed.width[l - 1] + ed.width[l];
+        G.off[e] = off;
+        off += train_grad_partials(ed, na[e]);
+        if (na[e] > 0)
+            shm = std::max(shm, (size_t)G.stride[e] * G.apb[e]
+                                * sizeof(double));
+        nb = std::max(nb, G.nb[e]);
+        nw = std::max(nw, G.nw[e]);
     }
-    int const per = (int)train_lds_per_atom(ed);
-    int const apb = train_atoms_per_grad_block(ed);
-    int const nb = (na + apb - 1) / apb;
-    size_t const shm = (size_t)per * apb * sizeof(double);
-    k_train_grad<<<nb, 64, shm, s>>>(A, e, atoms, na, per, apb, part, nw);
-    k_train_reduce<<<(nw + 255) / 256, 256, 0, s>>>(part, nb, nw, grad);
+    if (nb > 0)
+        k_train_grad<<<dim3(nb, A.T.ne), kGradThreads, shm, s>>>(A, G, part);
+    k_train_reduce<<<dim3((nw + 255) / 256, A.T.ne), 256, 0, s>>>(G, A.T,
+                                                                 part, grad);
     return hipGetLastError();
 }
 
