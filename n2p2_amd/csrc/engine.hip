@@ -115,6 +115,8 @@ struct hdnnp_ctx
     DBuf<ScaleDesc> dScale;
     DBuf<CompGroup> dCompGroup;
     DBuf<CompMember> dCompMember;
+    DBuf<CompRun> dCompRun;
+    DBuf<CompAng> dCompAng;
     DBuf<int> dPairGroups, dPairCount;
     DBuf<double> dWeights;
     DBuf<float> dWeights32;
@@ -362,6 +364,8 @@ struct hdnnp_ctx
         up(dScale, flat.scale);
         up(dCompGroup, flat.cgroup);
         up(dCompMember, flat.cmember);
+        up(dCompRun, flat.crun);
+        up(dCompAng, flat.cang);
         up(dPairGroups, flat.pairGroups);
         up(dPairCount, flat.pairCount);
         up(dWeights, flat.weights);
@@ -398,10 +402,16 @@ struct hdnnp_ctx
         T.weights32 = dWeights32.p;
         T.cgroup = dCompGroup.p;
         T.cmember = dCompMember.p;
+        T.crun = dCompRun.p;
+        T.cang = dCompAng.p;
         T.ncgroup = (int)flat.cgroup.size();
-        T.maxCompMembers = 1;
+        T.maxCompMembers = T.maxCompRuns = T.maxCompAngs = 1;
         for (auto const& g : flat.cgroup)
+        {
             T.maxCompMembers = std::max(T.maxCompMembers, g.nmem);
+            T.maxCompRuns = std::max(T.maxCompRuns, g.nrun);
+            T.maxCompAngs = std::max(T.maxCompAngs, g.nang);
+        }
         ld = std::max(1, T.maxnsf);
         maxMembers = 0;
         maxCfg = 1;
@@ -1436,6 +1446,7 @@ void hdnnp_ctx_destroy(hdnnp_ctx* c)
     c->dElem.release(); c->dCfg.release(); c->dGroup.release();
     c->dMember.release(); c->dRun.release(); c->dScale.release(); c->dPairGroups.release();
     c->dCompGroup.release(); c->dCompMember.release();
+    c->dCompRun.release(); c->dCompAng.release();
     c->dPairCount.release(); c->dWeights.release();
     c->dWeights32.release();
     for (auto& b : c->dAtomsOfElem) b.release();

@@ -866,6 +866,8 @@ Model::Flat Model::flatten(int chunk) const
             cg.e2 = sf_radial(g.type) ? -1 : g.e2;
             cg.nmem = (int)mem.size();
             cg.mem0 = (int)F.cmember.size();
+            cg.run0 = (int)F.crun.size();
+            cg.ang0 = (int)F.cang.size();
             cg.rmax = 0.0;
             for (size_t q = 0; q < mem.size(); ++q)
             {
@@ -875,18 +877,53 @@ Model::Flat Model::flatten(int chunk) const
                 cm.rc = s.rc;
                 cm.rcenter = (s.rc + s.rl) / 2.0;       // setLeftRight
                 cm.rscale = 1.0 / ((s.rc - s.rl) / 2.0);
-                // angleLeft * M_PI / 180.0 as SymFncBaseCompAng.cpp:106-108
-                cm.al = s.angleLeft * M_PI / 180.0;
-                cm.ar = s.angleRight * M_PI / 180.0;
-                cm.acenter = (cm.ar + cm.al) / 2.0;
-                cm.ascale = 1.0 / ((cm.ar - cm.al) / 2.0);
                 cm.sfac = s.scalingFactor;
                 cm.core = s.core;
                 cm.asym = s.asym ? 1 : 0;
                 cm.sf = s.index;
-                cm.newrad = (q == 0 || e.sf[mem[q - 1]].rc != s.rc
-                             || e.sf[mem[q - 1]].rl != s.rl) ? 1 : 0;
                 cg.rmax = std::max(cg.rmax, s.rc);
+                if (!sf_radial(g.type))
+                {
+                    // angleLeft * M_PI / 180.0 as
+                    // SymFncBaseCompAng.cpp:106-108
+                    CompAng ca{};
+                    ca.al = s.angleLeft * M_PI / 180.0;
+                    ca.ar = s.angleRight * M_PI / 180.0;
+                    ca.acenter = (ca.ar + ca.al) / 2.0;
+                    ca.ascale = 1.0 / ((ca.ar - ca.al) / 2.0);
+                    ca.core = s.core;
+                    while (cm.ang < cg.nang)
+                    {
+                        CompAng const& o = F.cang[cg.ang0 + cm.ang];
+                        if (o.al == ca.al && o.ar == ca.ar
+                            && o.core == ca.core) break;
+                        ++cm.ang;
+                    }
+                    if (cm.ang == cg.nang)
+                    {
+                        F.cang.push_back(ca);
+                        ++cg.nang;
+                    }
+                    CompRun const* prev = q ? &F.crun.back() : nullptr;
+                    bool const sameRad = prev && prev->rl == cm.rl
+                                      && prev->rc == cm.rc;
+                    if (!sameRad || prev->core != cm.core
+                        || prev->asym != cm.asym)
+                    {
+                        CompRun u{};
+                        u.rl = cm.rl;
+                        u.rc = cm.rc;
+                        u.rcenter = cm.rcenter;
+                        u.rscale = cm.rscale;
+                        u.core = cm.core;
+                        u.asym = cm.asym;
+                        u.m0 = (int)q;
+                        u.carry = sameRad && (g.type == 21 || g.type == 24);
+                        F.crun.push_back(u);
+                        ++cg.nrun;
+                    }
+                    F.crun.back().mend = (int)q + 1;
+                }
                 F.cmember.push_back(cm);
             }
             F.cgroup.push_back(cg);

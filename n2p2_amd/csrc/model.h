@@ -96,6 +96,8 @@ public:
         std::vector<ScaleDesc>  scale;
         std::vector<CompGroup>  cgroup;
         std::vector<CompMember> cmember;
+        std::vector<CompRun>    crun;
+        std::vector<CompAng>    cang;
         std::vector<int>        pairGroups, pairCount;
         std::vector<double>     weights;
     };

@@ -62,9 +62,8 @@ constexpr bool sf_weighted(int type)
 }
 
 // Members per compact group (SymGrpComp*: all compact SFs of one type and
-// centre / neighbour elements).  The compact kernels keep one row of member
-// sums per lane in LDS, T.maxCompMembers doubles wide; 96 members fill
-// 48 KiB of the 64 KiB a workgroup may use.
+// centre / neighbour elements); larger groups are rejected when the model
+// loads.
 constexpr int kMaxCompMembers = 96;
 
 struct CutCfg
@@ -123,20 +122,39 @@ struct MemberDesc
     int    level;     // zeta = 2^level (integer power), else -1
 };
 
-// A compact group's member: open radial interval (rl, rc) with its compact
-// function (x - center) * scale, and for the angular types the open angle
-// interval (al, ar) in radians with its compact function
-// (CompactFunction.cpp:57-72, SymFncBaseCompAng.cpp:57-110).
+// A compact group's member: its radial function, (x - center) scale on the
+// open interval (rl, rc) (CompactFunction.cpp:57-72); for the angular types
+// the members share these through the group's runs, and `ang` is the angle
+// function.
 struct CompMember
 {
     double rl, rc, rcenter, rscale;
-    double al, ar, acenter, ascale;
     double sfac;      // scalingFactor
     int    core;      // CT_POLY1..CT_POLY4 or CT_EXP (CoreFunction type)
     int    asym;      // asymmetric radial core (subtype "p?a")
     int    sf;        // SF index within the centre element
-    int    newrad;    // (rl, rc) differ from the previous member's
-                      // (calculateComp of SymGrpCompAngn.cpp:98-112)
+    int    ang;       // angle function (local to the group)
+};
+
+// Consecutive members of an angular compact group with one radial function.
+struct CompRun
+{
+    double rl, rc, rcenter, rscale;
+    int    core, asym;
+    int    m0, mend;  // members (local to the group)
+    int    carry;     // narrow types: (rl, rc) equal the previous run's, with
+                      // another core: its members take over cr(r_jk) of the
+                      // member before (calculateComp of
+                      // SymGrpCompAngn.cpp:98-112)
+    int    pad;
+};
+
+// Angle function on the open interval (al, ar) in radians
+// (SymFncBaseCompAng.cpp:57-110).
+struct CompAng
+{
+    double al, ar, acenter, ascale;
+    int    core, pad;
 };
 
 struct CompGroup
@@ -144,6 +162,8 @@ struct CompGroup
     int    type;      // 20-25
     int    e1, e2;    // neighbour elements (-1 where not used)
     int    nmem, mem0;
+    int    nrun, run0;    // angular: runs and angle functions
+    int    nang, ang0;
     int    pad;
     double rmax;      // largest member rc
 };
@@ -201,6 +221,10 @@ struct ModelTables
     const CompMember* cmember;
     int               ncgroup;      // compact groups over all elements
     int               maxCompMembers;   // largest compact group (>= 1)
+    const CompRun*    crun;
+    const CompAng*    cang;
+    int               maxCompRuns;      // most runs and angle functions of an
+    int               maxCompAngs;      // angular compact group (>= 1)
 };
 
 }  // namespace hdnnp
