@@ -955,40 +955,47 @@ void computeNN(hdnnp_ctx* c, bool deriv)
     int const n = (int)c->n;
     c->dE.ensure(n);
     c->dEdG.ensure((size_t)n * c->ld);
+    NNArgs a{};
+    a.T = c->T;
+    a.eds = c->flat.elem.data();
+    a.mode = c->precision == HDNNP_PRECISION_MIXED_BF16 ? 3
+           : c->precision == HDNNP_PRECISION_MIXED16 ? 2
+           : c->precision == HDNNP_PRECISION_MIXED ? 1 : 0;
+    a.tiles = c->nnTiles;
+    a.G = c->dG.p;
+    a.ldG = c->ld;
+    a.E = c->dE.p;
+    a.dEdG = c->dEdG.p;
+    a.deriv = deriv ? 1 : 0;
+    // Networks whose tile does not fit the LDS take the per-atom kernel.
+    NNArgs wide = a;
     size_t need = 0;
-    for (size_t e = 0; e < c->flat.elem.size(); ++e)
+    for (int e = 0; e < c->T.ne; ++e)
     {
-        int plane = 0;
-        for (int l = 1; l < c->flat.elem[e].nlayers; ++l)
-            plane += c->flat.elem[e].width[l];
-        need = std::max(need, (size_t)plane * 3 * c->hAtomsOfElem[e].size());
+        ElemDesc const& ed = c->flat.elem[e];
+        int const na = (int)c->hAtomsOfElem[e].size();
+        bool const fits = nn_mfma_lds_bytes(ed, a.mode, 1) <= 65536;
+        NNArgs& x = fits ? a : wide;
+        x.atoms[e] = c->dAtomsOfElem[e].p;
+        x.na[e] = na;
+        if (fits)
+            while (a.tiles > 1
+                   && nn_mfma_lds_bytes(ed, a.mode, a.tiles) > 65536)
+                a.tiles /= 2;
+        else
+        {
+            int plane = 0;
+            for (int l = 1; l < ed.nlayers; ++l) plane += ed.width[l];
+            need = std::max(need, (size_t)plane * 3 * na);
+        }
     }
     c->dScratch.ensure(need);
+    wide.scratch = c->dScratch.p;
     hipEvent_t ev = nullptr;
     c->begin(K_NETWORK, ev);
-    for (size_t e = 0; e < c->flat.elem.size(); ++e)
-    {
-        NNArgs a{};
-        a.T = c->T;
-        a.ed = c->flat.elem[e];
-        a.mode = c->precision == HDNNP_PRECISION_MIXED_BF16 ? 3
-               : c->precision == HDNNP_PRECISION_MIXED16 ? 2
-               : c->precision == HDNNP_PRECISION_MIXED ? 1 : 0;
-        a.tiles = c->nnTiles;
-        while (a.tiles > 1 && nn_mfma_lds_bytes(a.ed, a.mode, a.tiles) > 65536)
-            a.tiles /= 2;
-        if (nn_mfma_lds_bytes(a.ed, a.mode, 1) > 65536) a.mode = -1;
-        a.e = (int)e;
-        a.atoms = c->dAtomsOfElem[e].p;
-        a.na = (int)c->hAtomsOfElem[e].size();
-        a.G = c->dG.p;
-        a.ldG = c->ld;
-        a.E = c->dE.p;
-        a.dEdG = c->dEdG.p;
-        a.scratch = c->dScratch.p;
-        a.deriv = deriv ? 1 : 0;
-        hipCheck(launch_nn(a, c->stream), "networks");
-    }
+    hipCheck(launch_nn(a, c->stream), "networks");
+    for (int e = 0; e < c->T.ne; ++e)
+        hipCheck(launch_nn_atoms(wide, e, c->stream), "networks");
     c->end(K_NETWORK, ev);
     c->haveNN = true;
     c->haveNNDeriv = deriv;

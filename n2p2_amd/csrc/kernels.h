@@ -221,28 +221,33 @@ hipError_t launch_force_gather(int n, const int* off, const int* cnt,
                                const int* order, int mode, int64_t nslots,
                                double* F, hipStream_t s);
 
-// Atomic networks for the atoms of one element.  mode -1: per-atom FP64
-// kernel (any width); 0: FP64 MFMA tiles; 1: FP32 MFMA tiles; 2 / 3: FP16 /
+// Atomic networks, all elements in one launch.  mode
+// 0: FP64 MFMA tiles; 1: FP32 MFMA tiles; 2 / 3: FP16 /
 // BF16 MFMA tiles (hi + lo operand split) with FP32 accumulation.  The MFMA
-// kernels run `tiles` (1, 2 or 4) tiles of 16 atoms per wave and need
+// kernels run `tiles` (1, 2 or 4) tiles of 16 atoms per workgroup and need
 // nn_mfma_lds_bytes(ed, mode, tiles) of LDS.
 struct NNArgs
 {
     ModelTables T;
-    ElemDesc ed;                 // host copy of T.elem[e]
-    int mode;
-    int e;                       // element
-    const int* atoms;            // atom indices of element e
-    int na;
+    const ElemDesc* eds;    // host copy of the element descriptors
+    int mode;               // 0 FP64, 1 FP32, 2 FP16, 3 BF16 MFMA
+    int tiles;              // 16-atom tiles per workgroup: 1, 2 or 4
+    // Per element its atoms; elements with none, or whose networks are too
+    // wide for the MFMA kernel, have na = 0 there.  blk0: first workgroup of
+    // each element (set by launch_nn).
+    const int* atoms[kMaxElements];
+    int na[kMaxElements];
+    int blk0[kMaxElements + 1];
     const double* G;
     int ldG;
-    double* E;                   // per atom energy (indexed by atom)
-    double* dEdG;                // n x ldG (indexed by atom)
-    double* scratch;             // sum(width[l]) * 3 * na doubles
+    double* E;
+    double* dEdG;
+    double* scratch;        // launch_nn_atoms
     int deriv;
-    int tiles;                   // 16-atom tiles per wave (MFMA modes)
 };
-hipError_t launch_nn(NNArgs const& a, hipStream_t s);
+hipError_t launch_nn(NNArgs& a, hipStream_t s);
+// The per-atom FP64 kernel for element e (networks too wide for MFMA tiles).
+hipError_t launch_nn_atoms(NNArgs const& a, int e, hipStream_t s);
 size_t nn_mfma_lds_bytes(ElemDesc const& ed, int mode, int tiles);
 
 hipError_t launch_energy_sum(const double* E, int n, double* out, hipStream_t s);

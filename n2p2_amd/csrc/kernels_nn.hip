@@ -12,18 +12,20 @@
 #include "device_common.h"
 #include "kernels.h"
 
+#include <algorithm>
+
 namespace hdnnp {
 
 namespace {
 
-__global__ __launch_bounds__(256) void k_nn(NNArgs a)
+__global__ __launch_bounds__(256) void k_nn(NNArgs a, int e)
 {
     int const t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= a.na) return;
+    if (t >= a.na[e]) return;
     ModelTables const& T = a.T;
-    ElemDesc const& ed = T.elem[a.e];
-    int const atom = a.atoms[t];
-    int const na = a.na;
+    ElemDesc const& ed = T.elem[e];
+    int const atom = a.atoms[e][t];
+    int const na = a.na[e];
     int const L = ed.nlayers;
     double const* __restrict__ Gi = a.G + (size_t)atom * a.ldG;
     // scratch: value, dfdx and delta planes, each sum(width[1..L-1]) x na
@@ -102,7 +104,7 @@ __global__ __launch_bounds__(256) void k_nn(NNArgs a)
     }
 }
 
-// Matrix-core (MFMA) form of the same networks: one wavefront per tile of
+// Matrix-core (MFMA) form of the same networks: one workgroup per tile of
 // 16 atoms of one element; every layer is the GEMM Z = X W^T over the tile
 // (K = fan-in), the backward pass the GEMMs Delta_(l-1) = Delta_l W_l
 // (K = fan-out).  Activations and derivatives live in LDS per tile, each
@@ -143,7 +145,8 @@ template <> struct NNMma<0>
     __device__ static double a(Act const* X, int ld, int nk, int k0, int lane)
     {
         int const m = lane & 15, k = k0 + (lane >> 4);
-        return k < nk ? X[m * ld + k] : 0.0;
+        double const x = X[m * ld + min(k, nk - 1)];
+        return k < nk ? x : 0.0;
     }
     // B element (k, j) = W[j * ldw + k] (forward: W^T) or W[k * ldw + j]
     // (backward); zero outside [0, nk) x [0, nj).
@@ -152,8 +155,10 @@ template <> struct NNMma<0>
                                int lane)
     {
         int const j = j0 + (lane & 15), k = k0 + (lane >> 4);
-        if (k >= nk || j >= nj) return 0.0;
-        return T.weights[off + (trans ? j * ldw + k : k * ldw + j)];
+        int const jc = min(j, nj - 1), kc = min(k, nk - 1);
+        double const x = T.weights[off + (trans ? jc * ldw + kc
+                                                : kc * ldw + jc)];
+        return k < nk && j < nj ? x : 0.0;
     }
     __device__ static Acc mma(double a, double b, Acc c)
     {
@@ -170,15 +175,18 @@ template <> struct NNMma<1>
     __device__ static float a(Act const* X, int ld, int nk, int k0, int lane)
     {
         int const m = lane & 15, k = k0 + (lane >> 4);
-        return k < nk ? X[m * ld + k] : 0.0f;
+        float const x = X[m * ld + min(k, nk - 1)];
+        return k < nk ? x : 0.0f;
     }
     __device__ static float b(ModelTables const& T, int off, bool trans,
                               int ldw, int nk, int nj, int k0, int j0,
                               int lane)
     {
         int const j = j0 + (lane & 15), k = k0 + (lane >> 4);
-        if (k >= nk || j >= nj) return 0.0f;
-        return T.weights32[off + (trans ? j * ldw + k : k * ldw + j)];
+        int const jc = min(j, nj - 1), kc = min(k, nk - 1);
+        float const x = T.weights32[off + (trans ? jc * ldw + kc
+                                                 : kc * ldw + jc)];
+        return k < nk && j < nj ? x : 0.0f;
     }
     __device__ static Acc mma(float a, float b, Acc c)
     {
@@ -229,7 +237,8 @@ template <> struct NNMma<2>
         for (int q = 0; q < 4; ++q)
         {
             _Float16 h, l;
-            split_f16(k + q < nk ? X[m * ld + k + q] : 0.0f, h, l);
+            float const x = X[m * ld + min(k + q, nk - 1)];
+            split_f16(k + q < nk ? x : 0.0f, h, l);
             v.hi[q] = h;
             v.lo[q] = l;
         }
@@ -243,10 +252,10 @@ template <> struct NNMma<2>
 #pragma unroll
         for (int q = 0; q < 4; ++q)
         {
-            float w = 0.0f;
-            if (k + q < nk && j < nj)
-                w = T.weights32[off + (trans ? j * ldw + k + q
-                                             : (k + q) * ldw + j)];
+            int const jc = min(j, nj - 1), kc = min(k + q, nk - 1);
+            float w = T.weights32[off + (trans ? jc * ldw + kc
+                                               : kc * ldw + jc)];
+            if (k + q >= nk || j >= nj) w = 0.0f;
             _Float16 h, l;
             split_f16(w, h, l);
             v.hi[q] = h;
@@ -277,7 +286,8 @@ template <> struct NNMma<3>
         for (int q = 0; q < 4; ++q)
         {
             short h, l;
-            split_bf16(k + q < nk ? X[m * ld + k + q] : 0.0f, h, l);
+            float const x = X[m * ld + min(k + q, nk - 1)];
+            split_bf16(k + q < nk ? x : 0.0f, h, l);
             v.hi[q] = h;
             v.lo[q] = l;
         }
@@ -291,10 +301,10 @@ template <> struct NNMma<3>
 #pragma unroll
         for (int q = 0; q < 4; ++q)
         {
-            float w = 0.0f;
-            if (k + q < nk && j < nj)
-                w = T.weights32[off + (trans ? j * ldw + k + q
-                                             : (k + q) * ldw + j)];
+            int const jc = min(j, nj - 1), kc = min(k + q, nk - 1);
+            float w = T.weights32[off + (trans ? jc * ldw + kc
+                                               : kc * ldw + jc)];
+            if (k + q >= nk || j >= nj) w = 0.0f;
             short h, l;
             split_bf16(w, h, l);
             v.hi[q] = h;
@@ -312,10 +322,22 @@ template <> struct NNMma<3>
     __device__ static int row(int lane, int v) { return 4 * (lane >> 4) + v; }
 };
 
-// One wave computes R tiles of 16 atoms: every B operand (a weight tile)
-// is loaded once and used for the R tiles' MFMAs.
+// A workgroup computes R tiles of 16 atoms of one element; one launch covers
+// all elements (TAB.blk0).  Its waves split a layer's 16-neuron column tiles,
+// and every operand of a weight tile is loaded once for the R tiles, kUnroll
+// K steps ahead of the MFMAs that use them.
+//
+// Bound by latency: the layers follow one another, and a layer is a few
+// dependent steps of weight load, MFMA and activation.  With one wave per
+// tile, one K step in flight and one launch per element the networks took
+// 70 (FP64) and 63 us (mixed) on water boxes of 192 and 1,536 atoms whatever
+// their size, now 21 and 21; 512 B/C/N structures (130,842 atoms,
+// 102-30-30-1, mixed) 388 -> 264 us, 196,608 water atoms 198 -> 196 us (mixed)
+// and 327 -> 217 us (FP64).
+constexpr int kUnroll = 4;
+
 template <int MODE, int R>
-__global__ __launch_bounds__(64) void k_nn_mfma(NNArgs a)
+__global__ __launch_bounds__(256) void k_nn_mfma(NNArgs a)
 {
     typedef NNMma<MODE> MM;
     typedef typename MM::Act Act;
@@ -323,10 +345,15 @@ __global__ __launch_bounds__(64) void k_nn_mfma(NNArgs a)
     extern __shared__ double nnsm[];
     Act* const act = (Act*)nnsm;
     ModelTables const& T = a.T;
-    ElemDesc const& ed = T.elem[a.e];
+    int e = 0;
+    while (e + 1 < T.ne && (int)blockIdx.x >= a.blk0[e + 1]) ++e;
+    ElemDesc const& ed = T.elem[e];
+    int const* __restrict__ atoms = a.atoms[e];
+    int const na = a.na[e];
     int const L = ed.nlayers;
-    int const lane = threadIdx.x;
-    int const tile0 = blockIdx.x * 16 * R;
+    int const tid = threadIdx.x, nthr = blockDim.x;
+    int const lane = tid & 63, w = uniform(tid >> 6), nw = nthr >> 6;
+    int const tile0 = ((int)blockIdx.x - a.blk0[e]) * 16 * R;
     // LDS per tile: value planes of layers 0..L-1, then derivative planes
     // of 1..L-1, each [16][width]; tile r at r * tstride.
     int voff[kMaxLayers], doff[kMaxLayers];
@@ -340,40 +367,52 @@ __global__ __launch_bounds__(64) void k_nn_mfma(NNArgs a)
     // Input layer: the tiles' scaled SFs (zero rows past the last atom).
     {
         int const nin = ed.width[0];
-        for (int q = lane; q < 16 * R * nin; q += 64)
+        for (int q = tid; q < 16 * R * nin; q += nthr)
         {
             int const m = q / nin, k = q - m * nin;
             int const t = tile0 + m;
             double g = 0.0;
-            if (t < a.na) g = a.G[(size_t)a.atoms[t] * a.ldG + k];
+            if (t < na) g = a.G[(size_t)atoms[t] * a.ldG + k];
             act[(m >> 4) * tstride + voff[0] + (m & 15) * nin + k] = (Act)g;
         }
     }
     __syncthreads();
+    // acc[r] = sum over k < nk of X_r[m][k] B[k][j], j in the tile at j0.
+    auto product = [&](Act const* X, int nk, int woff, bool trans, int ldw,
+                       int nj, int j0, Acc (&acc)[R]) {
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) acc[r][v] = 0;
+        for (int k0 = 0; k0 < nk; k0 += kUnroll * MM::K)
+        {
+            decltype(MM::b(T, 0, true, 0, 0, 0, 0, 0, 0)) b[kUnroll];
+#pragma unroll
+            for (int u = 0; u < kUnroll; ++u)
+                b[u] = MM::b(T, woff, trans, ldw, nk, nj, k0 + u * MM::K, j0,
+                             lane);
+#pragma unroll
+            for (int u = 0; u < kUnroll; ++u)
+                if (k0 + u * MM::K < nk)
+#pragma unroll
+                    for (int r = 0; r < R; ++r)
+                        acc[r] = MM::mma(MM::a(X + r * tstride, nk, nk,
+                                               k0 + u * MM::K, lane),
+                                         b[u], acc[r]);
+        }
+    };
     for (int l = 1; l < L; ++l)
     {
         int const nin = ed.width[l - 1], nout = ed.width[l];
-        for (int j0 = 0; j0 < nout; j0 += 16)
+        for (int j0 = 16 * w; j0 < nout; j0 += 16 * nw)
         {
-            Acc acc[R];
-#pragma unroll
-            for (int r = 0; r < R; ++r)
-#pragma unroll
-                for (int v = 0; v < 4; ++v) acc[r][v] = 0;
-            for (int k0 = 0; k0 < nin; k0 += MM::K)
-            {
-                auto const b = MM::b(T, ed.woff[l], true, nin, nin, nout, k0,
-                                     j0, lane);
-#pragma unroll
-                for (int r = 0; r < R; ++r)
-                    acc[r] = MM::mma(MM::a(act + r * tstride + voff[l - 1],
-                                           nin, nin, k0, lane),
-                                     b, acc[r]);
-            }
             int const j = j0 + (lane & 15);
+            double const bias = T.weights[ed.boff[l] + min(j, nout - 1)];
+            Acc acc[R];
+            product(act + voff[l - 1], nin, ed.woff[l], true, nin, nout, j0,
+                    acc);
             if (j < nout)
             {
-                double const bias = T.weights[ed.boff[l] + j];
 #pragma unroll
                 for (int r = 0; r < R; ++r)
 #pragma unroll
@@ -388,8 +427,8 @@ __global__ __launch_bounds__(64) void k_nn_mfma(NNArgs a)
                         P[voff[l] + m * nout + j] = (Act)val;
                         P[doff[l] + m * nout + j] = (Act)d;
                         int const t = tile0 + 16 * r + m;
-                        if (l == L - 1 && t < a.na)
-                            a.E[a.atoms[t]] = val;   // one output neuron
+                        if (l == L - 1 && t < na)
+                            a.E[atoms[t]] = val;   // one output neuron
                     }
             }
         }
@@ -397,34 +436,23 @@ __global__ __launch_bounds__(64) void k_nn_mfma(NNArgs a)
     }
     if (!a.deriv) return;
     // Output delta (one neuron): f' / fan-in with normalize_nodes.
-    for (int q = lane; q < 16 * R; q += 64)
+    if (ed.normalize)
     {
-        Act* const P = act + (q >> 4) * tstride + doff[L - 1];
-        double g = (double)P[q & 15];
-        if (ed.normalize) g /= ed.width[L - 2];
-        P[q & 15] = (Act)g;
+        for (int q = tid; q < 16 * R; q += nthr)
+        {
+            Act* const P = act + (q >> 4) * tstride + doff[L - 1];
+            P[q & 15] = (Act)((double)P[q & 15] / ed.width[L - 2]);
+        }
+        __syncthreads();
     }
-    __syncthreads();
     for (int l = L - 1; l >= 1; --l)
     {
         int const nin = ed.width[l - 1], nout = ed.width[l];
-        for (int j0 = 0; j0 < nin; j0 += 16)
+        for (int j0 = 16 * w; j0 < nin; j0 += 16 * nw)
         {
             Acc acc[R];
-#pragma unroll
-            for (int r = 0; r < R; ++r)
-#pragma unroll
-                for (int v = 0; v < 4; ++v) acc[r][v] = 0;
-            for (int k0 = 0; k0 < nout; k0 += MM::K)
-            {
-                auto const b = MM::b(T, ed.woff[l], false, nin, nout, nin, k0,
-                                     j0, lane);
-#pragma unroll
-                for (int r = 0; r < R; ++r)
-                    acc[r] = MM::mma(MM::a(act + r * tstride + doff[l], nout,
-                                           nout, k0, lane),
-                                     b, acc[r]);
-            }
+            product(act + doff[l], nout, ed.woff[l], false, nin, nin, j0,
+                    acc);
             int const j = j0 + (lane & 15);
             if (j < nin)
             {
@@ -443,13 +471,13 @@ __global__ __launch_bounds__(64) void k_nn_mfma(NNArgs a)
                             if (ed.normalize) g /= ed.width[l - 2];
                             act[q] = (Act)((double)acc[r][v] * g);
                         }
-                        else if (t < a.na)
-                            a.dEdG[(size_t)a.atoms[t] * a.ldG + j]
+                        else if (t < na)
+                            a.dEdG[(size_t)atoms[t] * a.ldG + j]
                                 = (double)acc[r][v];
                     }
             }
         }
-        __syncthreads();
+        if (l > 1) __syncthreads();
     }
 }
 
@@ -515,29 +543,61 @@ size_t nn_mfma_lds_bytes(ElemDesc const& ed, int mode, int tiles)
 
 namespace {
 
-template <int MODE>
-void launch_nn_tiles(NNArgs const& a, hipStream_t s)
+// Waves per workgroup.  Few workgroups (up to two per CU): as many as the
+// widest layer has column tiles, for latency.  Otherwise two, unless the tiles
+// are so small (16 workgroups or more fit a CU's LDS) that one wave each
+// fills the chip and the barriers only cost: 196,608 water atoms take 196,
+// 220 and 273 us with one, two and three waves (FP32), 306, 217 and 270 us
+// in FP64 (8 workgroups per CU); 512 B/C/N structures (FP32, 11 per CU) 337,
+// 264 and 332 us; 192 water atoms (FP64) 36, 24 and 21 us.
+int nn_waves(NNArgs const& a, int blocks, size_t shm)
 {
-    size_t const shm = nn_mfma_lds_bytes(a.ed, a.mode, a.tiles);
-    int const nb = (a.na + 16 * a.tiles - 1) / (16 * a.tiles);
-    if (a.tiles == 4) k_nn_mfma<MODE, 4><<<nb, 64, shm, s>>>(a);
-    else if (a.tiles == 2) k_nn_mfma<MODE, 2><<<nb, 64, shm, s>>>(a);
-    else k_nn_mfma<MODE, 1><<<nb, 64, shm, s>>>(a);
+    int tiles = 1;
+    for (int e = 0; e < a.T.ne; ++e)
+        for (int l = 0; l < a.eds[e].nlayers; ++l)
+            tiles = std::max(tiles, (a.eds[e].width[l] + 15) / 16);
+    if (blocks <= 512) return std::min(tiles, 4);
+    if (shm * 16 <= 163840 && blocks >= 16 * 256) return 1;
+    return std::min(tiles, 2);
+}
+
+template <int MODE>
+void launch_nn_tiles(NNArgs& a, hipStream_t s)
+{
+    size_t shm = 0;
+    int nb = 0;
+    for (int e = 0; e < a.T.ne; ++e)
+    {
+        a.blk0[e] = nb;
+        if (a.na[e] <= 0) continue;
+        shm = std::max(shm, nn_mfma_lds_bytes(a.eds[e], a.mode, a.tiles));
+        nb += (a.na[e] + 16 * a.tiles - 1) / (16 * a.tiles);
+    }
+    for (int e = a.T.ne; e <= kMaxElements; ++e) a.blk0[e] = nb;
+    if (nb == 0) return;
+    int const nt = 64 * nn_waves(a, nb, shm);
+    if (a.tiles == 4) k_nn_mfma<MODE, 4><<<nb, nt, shm, s>>>(a);
+    else if (a.tiles == 2) k_nn_mfma<MODE, 2><<<nb, nt, shm, s>>>(a);
+    else k_nn_mfma<MODE, 1><<<nb, nt, shm, s>>>(a);
 }
 
 }  // namespace
 
-hipError_t launch_nn(NNArgs const& a, hipStream_t s)
+hipError_t launch_nn(NNArgs& a, hipStream_t s)
 {
-    if (a.na <= 0) return hipSuccess;
-    if (a.mode >= 0 && a.tiles != 1 && a.tiles != 2 && a.tiles != 4)
+    if (a.tiles != 1 && a.tiles != 2 && a.tiles != 4)
         return hipErrorInvalidValue;
-    if (a.mode < 0)
-        k_nn<<<(a.na + 255) / 256, 256, 0, s>>>(a);
-    else if (a.mode == 3) launch_nn_tiles<3>(a, s);
+    if (a.mode == 3) launch_nn_tiles<3>(a, s);
     else if (a.mode == 2) launch_nn_tiles<2>(a, s);
     else if (a.mode == 1) launch_nn_tiles<1>(a, s);
     else launch_nn_tiles<0>(a, s);
+    return hipGetLastError();
+}
+
+hipError_t launch_nn_atoms(NNArgs const& a, int e, hipStream_t s)
+{
+    if (a.na[e] <= 0) return hipSuccess;
+    k_nn<<<(a.na[e] + 255) / 256, 256, 0, s>>>(a, e);
     return hipGetLastError();
 }
 
