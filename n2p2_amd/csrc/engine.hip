@@ -175,6 +175,9 @@ struct hdnnp_ctx
     DBuf<double> dScatF;
     DBuf<int> dCellOfAtom, dRank, dCellCount, dCellStart, dCellAtoms, dCount,
         dOff, dStats, dBlockSums, dTotal;
+    int* hStats = nullptr;      // pinned: flags and largest count of a build
+    bool ownOrder = false;      // gather in atom order (no dCellAtoms)
+    const int* atomOrder() const { return ownOrder ? nullptr : dCellAtoms.p; }
     DBuf<uint64_t> dKeys;
     DBuf<int> dNbrJ, dPartner;
     DBuf<double4> dGeo;
@@ -517,12 +520,110 @@ void launchPartner(hdnnp_ctx* c, int n)
     hipEvent_t ev = nullptr;
     c->begin(K_PARTNER, ev, c->side);
     hipCheck(launch_nl_partner(n, c->dOff.p, c->dCount.p, c->dKeys.p,
-                               c->dCellAtoms.p, c->dPartner.p, c->entryCap,
+                               c->atomOrder(), c->dPartner.p, c->entryCap,
                                c->side),
              "nl partner");
     c->end(K_PARTNER, ev, c->side);
     hipCheck(hipEventRecord(c->evPartnerDone, c->side), "hipEventRecord");
     c->partnerPending = true;
+}
+
+
+// The host's copy of a build's statistics: dStats is cleared when it is made
+// and by every read.
+void ensureStats(hdnnp_ctx* c)
+{
+    if (!c->hStats)
+        hipCheck(hipHostMalloc((void**)&c->hStats, 4 * sizeof(int), 0),
+                 "hipHostMalloc");
+    if (c->dStats.cap < 4)
+    {
+        c->dStats.ensure(4);
+        hipCheck(hipMemsetAsync(c->dStats.p, 0, 4 * sizeof(int), c->stream),
+                 "memset");
+    }
+}
+
+// hstat[0] = largest count, hstat[1..3] = the builder's flags (waits).
+void readStats(hdnnp_ctx* c, int* hstat)
+{
+    hipCheck(launch_list_stats(c->dCount.p, (int)c->n, c->dStats.p, c->hStats,
+                               c->stream), "list stats");
+    hipCheck(hipStreamSynchronize(c->stream), "sync");
+    for (int k = 0; k < 4; ++k) hstat[k] = c->hStats[k];
+}
+
+void ensureEntries(hdnnp_ctx* c, int64_t E)
+{
+    if (E < 0 || E > (int64_t)2000000000)
+        throw Error(HDNNP_E_CAPACITY, "ERROR: Neighbour list too large.\n");
+    c->dKeys.ensure(E);
+    c->dNbrJ.ensure(E);
+    c->dGeo.ensure(E);
+    c->dPartner.ensure(E);
+    c->entryCap = E;
+}
+
+// Slots per atom: 1/8 headroom over the largest count plus 16, a multiple of
+// 16.
+int slabFor(int maxc) { return ((maxc + maxc / 8 + 16) + 15) / 16 * 16; }
+
+BatchCell batchCell(double const box[3][3], double rc)
+{
+    BatchCell C{};
+    C.periodic = 1;
+    for (int k = 0; k < 3; ++k)
+        for (int q = 0; q < 3; ++q) C.box[k][q] = box[k][q];
+    inverseBox(C.box, C.invbox);
+    cellWidths(C.box, rc, C.proj, C.pbc);
+    return C;
+}
+
+// Lists by k_nl_batch into fixed per-atom slot ranges: one fill pass if the
+// ranges are known from a build of as many atoms, else (or on overflow) a
+// count pass first.  cells null: one structure in cell `one`.
+void fillSlabs(hdnnp_ctx* c, double rc, const BatchCell* cells,
+               BatchCell const& one)
+{
+    int const n = (int)c->n;
+    hipStream_t s = c->stream;
+    int hstat[4] = {0, 0, 0, 0};
+    auto fill = [&]() {
+        int64_t const E = std::max<int64_t>((int64_t)n * c->slab, 1);
+        ensureEntries(c, E);
+        if (cells)
+            hipCheck(launch_slab_starts(n, c->slab, c->dOff.p, s),
+                     "slab starts");
+        hipCheck(launch_nl_batch(1, n, rc, c->dR.p, c->dStructOf.p,
+                                 c->dStructOff.p, cells, one, c->dCount.p,
+                                 c->dStats.p, c->dOff.p, c->slab, c->dKeys.p,
+                                 c->dNbrJ.p, c->dGeo.p, s), "nl fill");
+        readStats(c, hstat);
+    };
+    bool built = false;
+    if (c->slab > 0 && c->slabAtoms == n)
+    {
+        fill();
+        built = hstat[3] == 0;
+    }
+    if (!built)
+    {
+        hipCheck(launch_nl_batch(0, n, rc, c->dR.p, c->dStructOf.p,
+                                 c->dStructOff.p, cells, one, c->dCount.p,
+                                 nullptr, nullptr, 0, nullptr, nullptr,
+                                 nullptr, s), "nl count");
+        readStats(c, hstat);
+        if (!cells && hstat[0] > 8192)
+            throw Error(HDNNP_E_CAPACITY,
+                        "ERROR: More than 8192 neighbours for one atom.\n");
+        c->slab = slabFor(hstat[0]);
+        c->slabAtoms = n;
+        fill();
+        if (hstat[3] != 0)
+            throw Error(HDNNP_E_DEVICE,
+                        "ERROR: Neighbour count changed between passes.\n");
+    }
+    c->maxNeigh = std::min(hstat[0], c->slab);
 }
 
 void buildBatchNeighborList(hdnnp_ctx* c, double rc)
@@ -536,13 +637,12 @@ void buildBatchNeighborList(hdnnp_ctx* c, double rc)
     for (int64_t st = 0; st < ns; ++st)
     {
         BatchCell& C = cells[st];
-        C = BatchCell{};
         if (!c->hPeriodic[st]) continue;
-        C.periodic = 1;
+        double box[3][3];
         for (int k = 0; k < 3; ++k)
-            for (int q = 0; q < 3; ++q) C.box[k][q] = c->hBoxes[9 * st + 3 * k + q];
-        inverseBox(C.box, C.invbox);
-        cellWidths(C.box, rc, C.proj, C.pbc);
+            for (int q = 0; q < 3; ++q)
+                box[k][q] = c->hBoxes[9 * st + 3 * k + q];
+        C = batchCell(box, rc);
         int64_t nimg = 1;
         for (int k = 0; k < 3; ++k)
         {
@@ -570,64 +670,56 @@ void buildBatchNeighborList(hdnnp_ctx* c, double rc)
     c->dCount.ensure(n);
     c->dOff.ensure(n + 1);
     c->dStats.ensure(4);
-    c->dBlockSums.ensure((n + 1023) / 1024 + 1);
-    c->dTotal.ensure(1);
-    hipCheck(hipMemsetAsync(c->dStats.p, 0, 4 * sizeof(int), s), "memset");
-    int hstat[4] = {0, 0, 0, 0};
-    auto readStats = [&]() {
-        hipCheck(hipMemcpyAsync(hstat, c->dStats.p, 4 * sizeof(int),
-                                hipMemcpyDeviceToHost, s), "stats");
-        hipCheck(hipStreamSynchronize(s), "sync");
-        hipCheck(hipMemsetAsync(c->dStats.p, 0, 4 * sizeof(int), s),
-                 "memset");
-    };
-    auto fill = [&]() {
-        if ((int64_t)n * c->slab > (int64_t)2000000000)
-            throw Error(HDNNP_E_CAPACITY,
-                        "ERROR: Neighbour list too large.\n");
-        int64_t const E = std::max<int64_t>((int64_t)n * c->slab, 1);
-        c->dKeys.ensure(E);
-        c->dNbrJ.ensure(E);
-        c->dGeo.ensure(E);
-        c->dPartner.ensure(E);
-        c->entryCap = E;
-        hipCheck(launch_slab_starts(n, c->slab, c->dOff.p, s), "slab starts");
-        hipCheck(launch_nl_batch(1, n, rc, c->dR.p, c->dStructOf.p,
-                                 c->dStructOff.p, c->dCells.p, c->dCount.p,
-                                 c->dStats.p, c->dOff.p, c->slab, c->dKeys.p,
-                                 c->dNbrJ.p, c->dGeo.p, s), "batch nl fill");
-        hipCheck(launch_max_int(c->dCount.p, n, c->dStats.p, s), "count max");
-        readStats();
-    };
-    bool built = false;
-    if (c->slab > 0 && c->slabAtoms == n)
-    {
-        fill();
-        built = hstat[3] == 0;
-    }
-    if (!built)
-    {
-        hipCheck(launch_nl_batch(0, n, rc, c->dR.p, c->dStructOf.p,
-                                 c->dStructOff.p, c->dCells.p, c->dCount.p,
-                                 nullptr, nullptr, 0, nullptr, nullptr,
-                                 nullptr, s), "batch nl count");
-        hipCheck(launch_max_int(c->dCount.p, n, c->dStats.p, s), "count max");
-        readStats();
-        int const maxc = hstat[0];
-        c->slab = ((maxc + maxc / 8 + 16) + 15) / 16 * 16;
-        c->slabAtoms = n;
-        fill();
-        if (hstat[3] != 0)
-            throw Error(HDNNP_E_DEVICE,
-                        "ERROR: Neighbour count changed between passes.\n");
-    }
+    ensureStats(c);
+    fillSlabs(c, rc, c->dCells.p, BatchCell{});
     c->end(K_NEIGHBOR, ev0);
+    c->ownOrder = true;
     launchPartner(c, n);
     c->slabLayout = true;
     c->Mvalid = false;
-    c->maxNeigh = std::min(hstat[0], c->slab);
     c->haveNL = true;
     c->haveSF = c->haveNN = c->haveNNDeriv = false;
+}
+
+// A single structure of at most kSmallList atoms without cells; false if it
+// is larger or needs too many images.
+bool buildSmallNeighborList(hdnnp_ctx* c, double rc)
+{
+    int const n = (int)c->n;
+    if (n > kSmallList) return false;
+    BatchCell one{};
+    c->pbc[0] = c->pbc[1] = c->pbc[2] = 0;
+    if (c->periodic)
+    {
+        one = batchCell(c->box, rc);
+        int64_t cand = n;
+        for (int k = 0; k < 3; ++k)
+        {
+            // As the cell path: no cell shorter than rc / 60.
+            if (!(std::ceil(rc / one.proj[k] * (1.0 + 1e-6)) <= 60.0))
+                return false;
+            c->pbc[k] = one.pbc[k];
+            cand *= 2 * one.pbc[k] + 1;
+        }
+        if (cand > (int64_t)1 << 22) return false;
+    }
+    hipEvent_t ev0 = nullptr;
+    c->begin(K_NEIGHBOR, ev0);
+    c->dCount.ensure(n);
+    c->dOff.ensure(n + 1);
+    ensureStats(c);
+    fillSlabs(c, rc, nullptr, one);
+    if (c->maxNeigh > 8192)
+        throw Error(HDNNP_E_CAPACITY,
+                    "ERROR: More than 8192 neighbours for one atom.\n");
+    c->end(K_NEIGHBOR, ev0);
+    c->ownOrder = true;
+    launchPartner(c, n);
+    c->slabLayout = true;
+    c->Mvalid = false;
+    c->haveNL = true;
+    c->haveSF = c->haveNN = c->haveNNDeriv = false;
+    return true;
 }
 
 void buildNeighborList(hdnnp_ctx* c, double rc)
@@ -640,6 +732,8 @@ void buildNeighborList(hdnnp_ctx* c, double rc)
         buildBatchNeighborList(c, rc);
         return;
     }
+    if (buildSmallNeighborList(c, rc)) return;
+    c->ownOrder = false;
     NLParams& p = c->nl;
     p = NLParams{};
     p.n = (int)c->n;
@@ -712,11 +806,10 @@ void buildNeighborList(hdnnp_ctx* c, double rc)
     c->dCellAtoms.ensure(n);
     c->dCount.ensure(n);
     c->dOff.ensure(n + 1);
-    c->dStats.ensure(4);
+    ensureStats(c);
     c->dBlockSums.ensure((std::max(n, ncell) + 1023) / 1024 + 1);
     c->dTotal.ensure(1);
     hipCheck(hipMemsetAsync(c->dCellCount.p, 0, ncell * sizeof(int), s), "memset");
-    hipCheck(hipMemsetAsync(c->dStats.p, 0, 4 * sizeof(int), s), "memset");
     hipCheck(launch_nl_bin(p, c->dR.p, c->dCellOfAtom.p, c->dRank.p,
                            c->dCellCount.p, s), "nl bin");
     hipCheck(scan_exclusive(c->dCellCount.p, c->dCellStart.p, ncell,
@@ -729,47 +822,22 @@ void buildNeighborList(hdnnp_ctx* c, double rc)
     bool cellKernels = (2 * p.m[0] + 1) * (2 * p.m[1] + 1) * (2 * p.m[2] + 1)
                      <= 64;
     int hstat[4] = {0, 0, 0, 0};
-    auto readStats = [&]() {
-        hipCheck(hipMemcpyAsync(hstat, c->dStats.p, 4 * sizeof(int),
-                                hipMemcpyDeviceToHost, s), "stats");
-        hipCheck(hipStreamSynchronize(s), "sync");
-    };
-    auto clearStats = [&]() {
-        hipCheck(hipMemsetAsync(c->dStats.p, 0, 4 * sizeof(int), s),
-                 "memset");
-    };
-    auto ensureEntries = [&](int64_t E) {
-        if (E < 0 || E > (int64_t)2000000000)
-            throw Error(HDNNP_E_CAPACITY,
-                        "ERROR: Neighbour list too large.\n");
-        c->dKeys.ensure(E);
-        c->dNbrJ.ensure(E);
-        c->dGeo.ensure(E);
-        c->dPartner.ensure(E);
-        c->entryCap = E;
-    };
-    auto slabFor = [](int maxc) {
-        // 1/8 headroom over the largest count plus 16, a multiple of 16.
-        return ((maxc + maxc / 8 + 16) + 15) / 16 * 16;
-    };
     bool built = false;
     if (cellKernels && c->slab > 0 && c->slabAtoms == n)
     {
         // Slab build: one pass, no count kernel.  The counts, their maximum
         // and an overflow flag come back with the fill; on overflow the
         // list is rebuilt below with a range sized by the new maximum.
-        ensureEntries((int64_t)n * c->slab);
+        ensureEntries(c, (int64_t)n * c->slab);
         hipCheck(launch_slab_starts(n, c->slab, c->dOff.p, s), "slab starts");
         hipCheck(launch_nl_fill_cell(p, ncell, c->dR.p, c->dCellStart.p,
                                      c->dCellCount.p, c->dCellAtoms.p,
                                      c->dCount.p, c->dStats.p, c->dOff.p,
                                      c->slab, c->dKeys.p, c->dNbrJ.p,
                                      c->dGeo.p, s), "nl fill");
-        hipCheck(launch_max_int(c->dCount.p, n, c->dStats.p, s), "count max");
-        readStats();
+        readStats(c, hstat);
         if (hstat[2] > 0) cellKernels = false;    // staging overflow
         else if (hstat[3] == 0) built = true;
-        clearStats();
     }
     int maxc = hstat[0];
     if (!built)
@@ -787,15 +855,11 @@ void buildNeighborList(hdnnp_ctx* c, double rc)
                                          c->dCellCount.p, c->dCellAtoms.p,
                                          c->dCount.p, c->dStats.p, s),
                          "nl count");
-            hipCheck(launch_max_int(c->dCount.p, n, c->dStats.p, s),
-                     "count max");
-            readStats();
+            readStats(c, hstat);
             if (!(cellKernels && hstat[2] > 0)) break;
             cellKernels = false;     // a cell overflowed the staging: redo
-            clearStats();
         }
         maxc = hstat[0];
-        clearStats();
         if (cellKernels)
         {
             c->slab = slabFor(maxc);
@@ -803,7 +867,7 @@ void buildNeighborList(hdnnp_ctx* c, double rc)
             if ((int64_t)n * c->slab > (int64_t)2000000000)
                 throw Error(HDNNP_E_CAPACITY,
                             "ERROR: Neighbour list too large.\n");
-            ensureEntries((int64_t)n * c->slab);
+            ensureEntries(c, (int64_t)n * c->slab);
             hipCheck(launch_slab_starts(n, c->slab, c->dOff.p, s),
                      "slab starts");
             hipCheck(launch_nl_fill_cell(p, ncell, c->dR.p, c->dCellStart.p,
@@ -811,8 +875,6 @@ void buildNeighborList(hdnnp_ctx* c, double rc)
                                          c->dCount.p, c->dStats.p, c->dOff.p,
                                          c->slab, c->dKeys.p, c->dNbrJ.p,
                                          c->dGeo.p, s), "nl fill");
-            hipCheck(launch_max_int(c->dCount.p, n, c->dStats.p, s),
-                     "count max");
         }
         else
         {
@@ -829,7 +891,7 @@ void buildNeighborList(hdnnp_ctx* c, double rc)
                 throw Error(HDNNP_E_CAPACITY,
                             "ERROR: More than 8192 neighbours for one "
                             "atom.\n");
-            ensureEntries(std::max(total, 1));
+            ensureEntries(c, std::max(total, 1));
             hipCheck(launch_nl_fill(p, c->dR.p, c->dElemAtom.p,
                                     c->dCellOfAtom.p, c->dCellStart.p,
                                     c->dCellCount.p, c->dCellAtoms.p,
@@ -1093,7 +1155,7 @@ void launchGather(hdnnp_ctx* c, int mode)
         c->begin(K_GATHER, ev2);
         hipCheck(launch_gather_md((int)c->n, c->dOff.p, m.skinCnt.p,
                                   m.newIdx.p, m.skinPartner.p, m.skinKeys.p,
-                                  c->dCslot.p, c->dCself.p, c->dCellAtoms.p,
+                                  c->dCslot.p, c->dCself.p, c->atomOrder(),
                                   mode, c->entryCap, c->dF.p, m.flags.p + 3,
                                   c->stream), "force gather (MD)");
         c->end(K_GATHER, ev2);
@@ -1104,7 +1166,7 @@ void launchGather(hdnnp_ctx* c, int mode)
         c->begin(K_GATHER, ev2);
         hipCheck(launch_force_gather((int)c->n, c->dOff.p, c->dCount.p,
                                      c->dNbrJ.p, c->dPartner.p, c->dCslot.p,
-                                     c->dCself.p, c->dCellAtoms.p, mode,
+                                     c->dCself.p, c->atomOrder(), mode,
                                      c->entryCap, c->dF.p, c->stream),
                  "force gather");
         c->end(K_GATHER, ev2);
@@ -1454,6 +1516,7 @@ void hdnnp_ctx_destroy(hdnnp_ctx* c)
     c->dMember.release(); c->dRun.release(); c->dScale.release(); c->dPairGroups.release();
     c->dCompGroup.release(); c->dCompMember.release();
     c->dCompRun.release(); c->dCompAng.release();
+    if (c->hStats) (void)hipHostFree(c->hStats);
     c->dPairCount.release(); c->dWeights.release();
     c->dWeights32.release();
     for (auto& b : c->dAtomsOfElem) b.release();
@@ -1928,22 +1991,17 @@ int hdnnp_set_structures(hdnnp_ctx* c, int64_t nstruct,
                 for (int q = 0; q < 9; ++q)
                     c->hBoxes[9 * s + q] = boxes[9 * s + q];
         }
-        std::vector<int> structOf((size_t)n), iota((size_t)n);
+        std::vector<int> structOf((size_t)n);
         for (int64_t s = 0; s < nstruct; ++s)
             for (int64_t i = atom_offsets[s]; i < atom_offsets[s + 1]; ++i)
                 structOf[i] = (int)s;
-        for (int64_t i = 0; i < n; ++i) iota[i] = (int)i;
         c->dStructOf.ensure(n);
         c->dStructOff.ensure(nstruct + 1);
-        c->dCellAtoms.ensure(n);
         hipCheck(hipMemcpy(c->dStructOf.p, structOf.data(), n * sizeof(int),
                            hipMemcpyHostToDevice), "structure index");
         hipCheck(hipMemcpy(c->dStructOff.p, c->hStructOff.data(),
                            (nstruct + 1) * sizeof(int),
                            hipMemcpyHostToDevice), "structure offsets");
-        // Atoms are gathered in their own order.
-        hipCheck(hipMemcpy(c->dCellAtoms.p, iota.data(), n * sizeof(int),
-                           hipMemcpyHostToDevice), "atom order");
     });
 }
 

@@ -51,7 +51,7 @@ hipError_t launch_nl_count_cell(NLParams const& p, int ncell, const double* r,
                                 hipStream_t s);
 // Writes atom i's entries from off[i] on, at most limit of them; count[i]
 // receives the true count, stats[3] = 1 if a count exceeds limit (the
-// largest count: launch_max_int over count).
+// largest count: launch_list_stats over count).
 hipError_t launch_nl_fill_cell(NLParams const& p, int ncell, const double* r,
                                const int* cellStart, const int* cellCount,
                                const int* cellAtoms, int* count, int* stats,
@@ -74,12 +74,21 @@ hipError_t launch_batch_extent(int nstruct, const double* r,
 // Batched structures: per-atom lists within each atom's structure
 // (structOf, structOff) over its cell's images.  mode 0 counts into count;
 // mode 1 writes at most `limit` entries per atom from off, stores count
-// and sets stats[3] on overflow (the largest count: launch_max_int).
+// and sets stats[3] on overflow (the largest count: launch_list_stats).
+// cells null: one structure of n atoms in cell `one` (the extent is found by
+// the kernel, off is written).
 hipError_t launch_nl_batch(int mode, int n, double rc, const double* r,
                            const int* structOf, const int* structOff,
-                           const BatchCell* cells, int* count, int* stats,
-                           const int* off, int limit, uint64_t* keys,
-                           int* nbrJ, double4* geo, hipStream_t s);
+                           const BatchCell* cells, BatchCell const& one,
+                           int* count, int* stats, int* off, int limit,
+                           uint64_t* keys, int* nbrJ, double4* geo,
+                           hipStream_t s);
+// Atoms up to which a single structure's list is built by k_nl_batch.
+constexpr int kSmallList = 2048;
+// host[0] = the largest count, host[1..3] = stats[1..3], which are cleared;
+// host is pinned memory.
+hipError_t launch_list_stats(const int* count, int n, int* stats, int* host,
+                             hipStream_t s);
 // --- Training of a radial-only model (kernels_train.hip)
 struct TrainArgs
 {

@@ -35,7 +35,7 @@ __global__ __launch_bounds__(256) void k_gather(
                 + (int)(threadIdx.x >> 6);
     int const lane = threadIdx.x & 63;
     if (t >= n) return;
-    int const i = order[t];
+    int const i = order ? order[t] : t;
     int const s0 = off[i], s1 = s0 + cnt[i];
     double fx = 0.0, fy = 0.0, fz = 0.0;
     for (int q = s0 + lane; q < s1; q += 64)

@@ -209,7 +209,7 @@ __global__ __launch_bounds__(256) void k_gather_md(
                 + (int)(threadIdx.x >> 6);
     int const lane = threadIdx.x & 63;
     if (t >= n) return;
-    int const i = order[t];
+    int const i = order ? order[t] : t;
     int const s0 = off[i], s1 = s0 + skinCnt[i];
     double fx = 0.0, fy = 0.0, fz = 0.0;
     for (int s = s0 + lane; s < s1; s += 64)

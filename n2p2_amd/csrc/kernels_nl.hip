@@ -281,7 +281,7 @@ __global__ __launch_bounds__(64) void k_nl(
 // limit of them (a fixed slot range per atom), stores the true count in
 // count[i] and sets stats[3] when a count exceeds limit (the host then
 // rebuilds with a larger range); the largest count comes from a reduction
-// over count[] afterwards (launch_max_int).
+// over count[] afterwards (launch_list_stats).
 constexpr int kCellCand = 1024;
 constexpr int kCellWaves = 4;
 
@@ -503,23 +503,18 @@ __global__ __launch_bounds__(256) void k_nl_cell(
     }
 }
 
-// Fractional extent of each periodic structure's atoms along its three
-// lattice directions (f = r invbox): the bounds the image pruning of
-// k_nl_batch uses.  One wave per structure.
-__global__ __launch_bounds__(64) void k_batch_extent(
-    int nstruct, const double* __restrict__ r,
-    const int* __restrict__ structOff, BatchCell* __restrict__ cells)
+// Fractional extent of the atoms [i0, i1) of a periodic structure along its
+// three lattice directions (f = r invbox): the bounds the image pruning of
+// k_nl_batch uses.  One wave; every lane gets the result.
+__device__ __forceinline__ void structure_extent(const double* __restrict__ r,
+                                                 int i0, int i1, BatchCell& C)
 {
-    int const st = blockIdx.x;
-    if (st >= nstruct) return;
-    BatchCell& C = cells[st];
-    if (!C.periodic) return;
-    int const lane = threadIdx.x;
     double lo[3] = {1e300, 1e300, 1e300}, hi[3] = {-1e300, -1e300, -1e300};
-    for (int i = structOff[st] + lane; i < structOff[st + 1]; i += 64)
+    for (int i = i0 + lane_id(); i < i1; i += 64)
     {
         double const x = r[3 * (size_t)i], y = r[3 * (size_t)i + 1],
                      z = r[3 * (size_t)i + 2];
+#pragma unroll
         for (int k = 0; k < 3; ++k)
         {
             double const f = x * C.invbox[0][k] + y * C.invbox[1][k]
@@ -528,6 +523,7 @@ __global__ __launch_bounds__(64) void k_batch_extent(
             hi[k] = fmax(hi[k], f);
         }
     }
+#pragma unroll
     for (int k = 0; k < 3; ++k)
     {
         for (int o = 32; o > 0; o >>= 1)
@@ -535,12 +531,27 @@ __global__ __launch_bounds__(64) void k_batch_extent(
             lo[k] = fmin(lo[k], __shfl_xor(lo[k], o));
             hi[k] = fmax(hi[k], __shfl_xor(hi[k], o));
         }
-        if (lane == 0)
-        {
-            C.fmin[k] = lo[k];
-            C.fmax[k] = hi[k];
-        }
+        C.fmin[k] = lo[k];
+        C.fmax[k] = hi[k];
     }
+}
+
+// The extents of a batch's structures, one wave each.
+__global__ __launch_bounds__(64) void k_batch_extent(
+    int nstruct, const double* __restrict__ r,
+    const int* __restrict__ structOff, BatchCell* __restrict__ cells)
+{
+    int const st = blockIdx.x;
+    if (st >= nstruct) return;
+    if (!cells[st].periodic) return;
+    BatchCell C = cells[st];
+    structure_extent(r, structOff[st], structOff[st + 1], C);
+    if (threadIdx.x == 0)
+        for (int k = 0; k < 3; ++k)
+        {
+            cells[st].fmin[k] = C.fmin[k];
+            cells[st].fmax[k] = C.fmax[k];
+        }
 }
 
 // Image range [lo, hi] along one lattice direction that can hold a
@@ -586,21 +597,49 @@ __device__ __forceinline__ void image_range(double f, double fmin,
 // places each lane's hits, in image order, behind those of the lanes
 // (atoms j) before it.  More images: candidates (j, image) in list order,
 // 64 per step, and a ballot compaction.
+//
+// A single structure of at most kSmallList atoms takes this kernel too
+// (cells null): its cell comes as an argument and every wave finds the
+// extent of the atoms itself, so that a build is this launch and the count
+// reduction.  Binning into cells needs eight more launches, its workgroups
+// are few, and the images of a cell below three cutoffs overflow their
+// staging, which then cost a count and a fill by the per-atom kernels.  List
+// builds including the host's wait, cells against this: 192 water atoms (27
+// images) 292 -> 62 us, 1,536 225 -> 100 us, 1,000 B/C/N atoms 202 -> 84 us.
+// The work grows as n^2: 2,000 B/C/N atoms take 123 us against the cells'
+// 131, 4,000 230 against 131 (water, wider cutoff: 129 against 168 and 200
+// against 182), hence the bound of 2,048.
 template <int MODE>
 __global__ __launch_bounds__(64) void k_nl_batch(
     int n, double rc2, double rcm, const double* __restrict__ r,
     const int* __restrict__ structOf, const int* __restrict__ structOff,
-    const BatchCell* __restrict__ cells, int* __restrict__ count,
-    int* __restrict__ stats, const int* __restrict__ off, int limit,
-    uint64_t* __restrict__ keysOut, int* __restrict__ nbrJ,
+    const BatchCell* __restrict__ cells, BatchCell one,
+    int* __restrict__ count, int* __restrict__ stats, int* __restrict__ off,
+    int limit, uint64_t* __restrict__ keysOut, int* __restrict__ nbrJ,
     double4* __restrict__ geo)
 {
     int const i = blockIdx.x;
     if (i >= n) return;
     int const lane = threadIdx.x;
-    int const st = structOf[i];
-    BatchCell const& C = cells[st];
-    int const a0 = structOff[st], na = structOff[st + 1] - a0;
+    int a0 = 0, na = n;
+    if (cells)
+    {
+        int const st = structOf[i];
+        one = cells[st];
+        a0 = structOff[st];
+        na = structOff[st + 1] - a0;
+    }
+    else
+    {
+        if (one.periodic) structure_extent(r, 0, n, one);
+        // The atom's slot range; the batch launch sets them beforehand.
+        if (MODE == 1 && lane == 0)
+        {
+            off[i] = i * limit;
+            if (i == n - 1) off[n] = n * limit;
+        }
+    }
+    BatchCell const& C = one;
     NLParams p{};
     for (int k = 0; k < 3; ++k)
         for (int c = 0; c < 3; ++c) p.box[k][c] = C.box[k][c];
@@ -623,7 +662,7 @@ __global__ __launch_bounds__(64) void k_nl_batch(
     float const invImg = 1.0f / (float)nimg, invW12 = 1.0f / (float)w12,
                 invW2 = 1.0f / (float)w2;
     int const total = na * nimg;
-    int const o = MODE == 1 ? off[i] : 0;
+    int const o = MODE == 1 ? (cells ? off[i] : i * limit) : 0;
     int hits = 0;
     if (nimg <= 64)
     {
@@ -773,7 +812,7 @@ __global__ __launch_bounds__(64) void k_partner(
 {
     int const w = xcd_work_index(blockIdx.x, gridDim.x);
     if (w >= n) return;
-    int const i = order[w];
+    int const i = order ? order[w] : w;
     int const s0 = off[i], s1 = s0 + cnt[i];
     uint64_t const first = (uint64_t)(uint32_t)i << 21;
     int a = s0, b = s1;
@@ -803,12 +842,10 @@ __global__ __launch_bounds__(64) void k_partner(
     }
 }
 
-// out[0] = max(in[0..n)) of non-negative counts; one block, fixed-order
-// tree (the per-atom neighbour counts, whose maximum sizes the fill's
-// LDS).  `in` is 16-byte aligned (a device allocation): four counts per
+// The largest of the non-negative counts in[0..n): one block, fixed-order
+// tree.  `in` is 16-byte aligned (a device allocation): four counts per
 // load, four loads in flight per thread.
-__global__ __launch_bounds__(1024) void k_max(const int* __restrict__ in,
-                                              int n, int* __restrict__ out)
+__device__ __forceinline__ int block_max(const int* __restrict__ in, int n)
 {
     __shared__ int s[1024];
     int const t = threadIdx.x;
@@ -829,7 +866,32 @@ __global__ __launch_bounds__(1024) void k_max(const int* __restrict__ in,
         if (t < o) s[t] = max(s[t], s[t + o]);
         __syncthreads();
     }
-    if (t == 0) out[0] = s[0];
+    return s[0];
+}
+
+// out[0] = the largest count.
+__global__ __launch_bounds__(1024) void k_max(const int* __restrict__ in,
+                                              int n, int* __restrict__ out)
+{
+    int const m = block_max(in, n);
+    if (threadIdx.x == 0) out[0] = m;
+}
+
+// What the host needs of a list build, in its own pinned memory (no copy
+// command): the largest count (its LDS capacity) and the builder's flags
+// stats[1..3], which are cleared for the next build.
+__global__ __launch_bounds__(1024) void k_list_stats(
+    const int* __restrict__ count, int n, int* __restrict__ stats,
+    int* __restrict__ host)
+{
+    int const m = block_max(count, n);
+    int const t = threadIdx.x;
+    if (t == 0) host[0] = m;
+    if (t > 0 && t < 4)
+    {
+        host[t] = stats[t];
+        stats[t] = 0;
+    }
 }
 
 // Exclusive scan helpers (block-level, then block offsets).
@@ -898,6 +960,13 @@ hipError_t scan_exclusive(const int* in, int* out, int n, int* blockSums,
 hipError_t launch_max_int(const int* in, int n, int* out, hipStream_t s)
 {
     k_max<<<1, 1024, 0, s>>>(in, n, out);
+    return hipGetLastError();
+}
+
+hipError_t launch_list_stats(const int* count, int n, int* stats, int* host,
+                             hipStream_t s)
+{
+    k_list_stats<<<1, 1024, 0, s>>>(count, n, stats, host);
     return hipGetLastError();
 }
 
@@ -978,20 +1047,21 @@ hipError_t launch_batch_extent(int nstruct, const double* r,
 
 hipError_t launch_nl_batch(int mode, int n, double rc, const double* r,
                            const int* structOf, const int* structOff,
-                           const BatchCell* cells, int* count, int* stats,
-                           const int* off, int limit, uint64_t* keys,
-                           int* nbrJ, double4* geo, hipStream_t s)
+                           const BatchCell* cells, BatchCell const& one,
+                           int* count, int* stats, int* off, int limit,
+                           uint64_t* keys, int* nbrJ, double4* geo,
+                           hipStream_t s)
 {
     if (n <= 0) return hipSuccess;
     double const rc2 = rc * rc, rcm = rc * (1.0 + 1e-6);
     if (mode == 0)
         k_nl_batch<0><<<n, 64, 0, s>>>(n, rc2, rcm, r, structOf, structOff,
-                                       cells, count, nullptr, nullptr, 0,
+                                       cells, one, count, nullptr, nullptr, 0,
                                        nullptr, nullptr, nullptr);
     else
         k_nl_batch<1><<<n, 64, 0, s>>>(n, rc2, rcm, r, structOf, structOff,
-                                       cells, count, stats, off, limit, keys,
-                                       nbrJ, geo);
+                                       cells, one, count, stats, off, limit,
+                                       keys, nbrJ, geo);
     return hipGetLastError();
 }
 
