@@ -176,6 +176,8 @@ struct hdnnp_ctx
     DBuf<int> dCellOfAtom, dRank, dCellCount, dCellStart, dCellAtoms, dCount,
         dOff, dStats, dBlockSums, dTotal;
     int* hStats = nullptr;      // pinned: flags and largest count of a build
+    double* hEnergy = nullptr;  // pinned: the last energy sum
+    DBuf<double> dSumScratch;
     bool ownOrder = false;      // gather in atom order (no dCellAtoms)
     const int* atomOrder() const { return ownOrder ? nullptr : dCellAtoms.p; }
     DBuf<uint64_t> dKeys;
@@ -1063,11 +1065,18 @@ void computeNN(hdnnp_ctx* c, bool deriv)
     c->haveNNDeriv = deriv;
 }
 
+// dst[0] (device) and host[0] (pinned, if not null) = sum of v[0..n).
+void sumOnDevice(hdnnp_ctx* c, double const* v, int n, double* dst,
+                 double* host)
+{
+    hipCheck(launch_energy_sum(v, n, c->dSumScratch.p, dst, host, c->stream),
+             "energy");
+}
+
 void launchEnergy(hdnnp_ctx* c)
 {
     c->dEnergy.ensure(1);
-    hipCheck(launch_energy_sum(c->dE.p, (int)c->n, c->dEnergy.p, c->stream),
-             "energy");
+    sumOnDevice(c, c->dE.p, (int)c->n, c->dEnergy.p, c->hEnergy);
 }
 
 double computeEnergy(hdnnp_ctx* c)
@@ -1076,12 +1085,9 @@ double computeEnergy(hdnnp_ctx* c)
         throw Error(HDNNP_E_INVALID, "ERROR: Networks not evaluated.\n");
     c->setDevice();
     launchEnergy(c);
-    double e = 0.0;
-    hipCheck(hipMemcpyAsync(&e, c->dEnergy.p, sizeof(double),
-                            hipMemcpyDeviceToHost, c->stream), "energy copy");
     c->sync();
-    c->energy = e;
-    return e;
+    c->energy = *c->hEnergy;
+    return c->energy;
 }
 
 void launchGather(hdnnp_ctx* c, int mode);
@@ -1494,6 +1500,12 @@ int hdnnp_ctx_create(const hdnnp_model* m, int device, hdnnp_ctx** out)
         hipCheck(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking),
                  "hipStreamCreate");
         c->uploadModel();
+        size_t const ns = energy_sum_scratch();
+        c->dSumScratch.ensure(ns);
+        hipCheck(hipMemsetAsync(c->dSumScratch.p, 0, ns * sizeof(double),
+                                c->stream), "memset");
+        hipCheck(hipHostMalloc((void**)&c->hEnergy, sizeof(double), 0),
+                 "hipHostMalloc");
         *out = c.release();
     });
 }
@@ -1517,6 +1529,8 @@ void hdnnp_ctx_destroy(hdnnp_ctx* c)
     c->dCompGroup.release(); c->dCompMember.release();
     c->dCompRun.release(); c->dCompAng.release();
     if (c->hStats) (void)hipHostFree(c->hStats);
+    if (c->hEnergy) (void)hipHostFree(c->hEnergy);
+    c->dSumScratch.release();
     c->dPairCount.release(); c->dWeights.release();
     c->dWeights32.release();
     for (auto& b : c->dAtomsOfElem) b.release();
@@ -2118,9 +2132,12 @@ int hdnnp_evaluate(hdnnp_ctx* c, int force_mode, double* energy)
         if (!c->externalNL) buildNeighborList(c, c->T.maxCutoff);
         computeSF(c, false);
         computeNN(c, force_mode >= 0);
-        double const e = computeEnergy(c);
-        if (force_mode >= 0) computeForces(c, force_mode);
-        if (energy) *energy = e;
+        // One wait for the energy and the forces together.
+        launchEnergy(c);
+        if (force_mode >= 0) computeForces(c, force_mode, false);
+        c->sync();
+        c->energy = *c->hEnergy;
+        if (energy) *energy = c->energy;
     });
 }
 
@@ -2436,7 +2453,7 @@ static double mtsRmse(hdnnp_ctx* sur)
     hipStream_t s = sur->stream;
     hipCheck(hipStreamSynchronize(S.full->stream), "sync");
     hipCheck(launch_md_fdiff2(n, sur->dF.p, S.full->dF.p, S.d2.p, s), "rmse");
-    hipCheck(launch_energy_sum(S.d2.p, n, S.sum.p, s), "rmse");
+    sumOnDevice(sur, S.d2.p, n, S.sum.p, nullptr);
     double v = 0.0;
     hipCheck(hipMemcpyAsync(&v, S.sum.p, sizeof(double),
                             hipMemcpyDeviceToHost, s), "rmse");
@@ -2733,7 +2750,7 @@ int hdnnp_train_gradient(hdnnp_ctx* c, const double* f_ref, double e_ref,
                                        c->tPart.p, c->tGrad.p, s),
                      "train gradient");
         }
-        hipCheck(launch_energy_sum(c->tD2.p, n, c->tLoss.p, s), "train loss");
+        sumOnDevice(c, c->tD2.p, n, c->tLoss.p, nullptr);
         double sumd2 = 0.0, energy = 0.0;
         hipCheck(hipMemcpyAsync(&sumd2, c->tLoss.p, sizeof(double),
                                 hipMemcpyDeviceToHost, s), "train loss");

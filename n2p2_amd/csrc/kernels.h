@@ -259,7 +259,11 @@ hipError_t launch_nn(NNArgs& a, hipStream_t s);
 hipError_t launch_nn_atoms(NNArgs const& a, int e, hipStream_t s);
 size_t nn_mfma_lds_bytes(ElemDesc const& ed, int mode, int tiles);
 
-hipError_t launch_energy_sum(const double* E, int n, double* out, hipStream_t s);
+// out[0] (device) and, if not null, host[0] (pinned memory) = sum of E[0..n);
+// scratch: energy_sum_scratch() doubles, zero at first.
+size_t energy_sum_scratch();
+hipError_t launch_energy_sum(const double* E, int n, double* scratch,
+                             double* out, double* host, hipStream_t s);
 
 // Unscaled-SF statistics for one element (min, max, sum, sum of squares)
 // over atoms of that element: out 4 x nsf.
