@@ -219,6 +219,23 @@ size_t force_backward_lds_bytes(int cap, int fp32);
 
 // Entries of atom i: [off[i], off[i] + cnt[i]).  order: the atoms sorted
 // by cell (processing order only).
+// A caller-given list of n centres and M entries (idx, elem, dr: the caller's
+// arrays) as the kernels read it; stats[1..3]: largest index, some index
+// negative, some element out of range.
+hipError_t launch_ext_entries(int n, int M, int ne, const int* idx,
+                              const int* elem, const double* dr, int* nbrJ,
+                              double4* geo, int* stats, hipStream_t s);
+// Most contributions to one target that launch_ext_sort takes.
+constexpr int kExtSort = 512;
+// count[b] (zero before) and rank[q] of the n + M contributions; then, with
+// start = exclusive scan of count, the table of k_scatter_ext.  idx may share
+// src: it is read before src is written.
+hipError_t launch_ext_count(int n, int M, const int* idx, const int* ctr,
+                            int* count, int* rank, hipStream_t s);
+hipError_t launch_ext_sort(int n, int M, int nt, const int* idx,
+                           const int* ctr, const int* off, const int* start,
+                           const int* count, const int* rank, uint64_t* keys,
+                           int64_t* srcOff, int* src, hipStream_t s);
 // Forces of a caller-given list onto the caller's atoms, in the order of
 // InterfaceLammps::getForces (k_scatter_ext).
 hipError_t launch_scatter_ext(int nt, const int64_t* srcOff, const int* src,

@@ -894,6 +894,103 @@ __global__ __launch_bounds__(1024) void k_list_stats(
     }
 }
 
+// --- Caller-given lists.  Entry q of centre i is the virtual atom n + q at
+// dr; its forces go to the caller's atom idx[q], the centre's own to ctr[i].
+
+// The list as the kernels read it, and its checks: stats[1] = largest caller
+// index, stats[2] = 1 if one is negative, stats[3] = 1 if an element is out
+// of range.
+__global__ __launch_bounds__(256) void k_ext_entries(
+    int n, int M, int ne, const int* __restrict__ idx,
+    const int* __restrict__ elem, const double* __restrict__ dr,
+    int* __restrict__ nbrJ, double4* __restrict__ geo, int* __restrict__ stats)
+{
+    int top = 0;
+    bool neg = false, bad = false;
+    for (int64_t q = (int64_t)blockIdx.x * 256 + threadIdx.x; q < M;
+         q += (int64_t)gridDim.x * 256)
+    {
+        int const b = idx[q], e = elem[q];
+        top = max(top, b);
+        neg |= b < 0;
+        bad |= e < 0 || e >= ne;
+        double const v[3] = {dr[3 * q], dr[3 * q + 1], dr[3 * q + 2]};
+        nbrJ[q] = n + (int)q;
+        geo[q] = make_double4(v[0], v[1], v[2], sqrt(norm2_pinned(v)));
+    }
+    // One atomic per block: all of them meet at one address.
+    __shared__ int tops[4];
+    for (int o = 32; o > 0; o >>= 1) top = max(top, __shfl_xor(top, o));
+    bool const anyNeg = __ballot(neg) != 0, anyBad = __ballot(bad) != 0;
+    if ((threadIdx.x & 63) == 0)
+    {
+        tops[threadIdx.x >> 6] = top;
+        if (anyNeg) atomicMax(stats + 2, 1);
+        if (anyBad) atomicMax(stats + 3, 1);
+    }
+    __syncthreads();
+    if (threadIdx.x == 0)
+        atomicMax(stats + 1, max(max(tops[0], tops[1]), max(tops[2], tops[3])));
+}
+
+// The contributions q < M (entries) and M + i (self forces) per target:
+// their number and, in arrival order, each one's rank.
+__global__ __launch_bounds__(256) void k_ext_count(
+    int n, int M, const int* __restrict__ idx, const int* __restrict__ ctr,
+    int* __restrict__ count, int* __restrict__ rank)
+{
+    int64_t const q = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (q >= (int64_t)M + n) return;
+    int const b = q < M ? idx[q] : ctr[q - M];
+    rank[q] = atomicAdd(count + b, 1);
+}
+
+// Their sort keys, target by target.  High half: 2 q + 1 for entry q and
+// 2 off[i] for the self force of centre i, the reference's loop order
+// (centres in order, each one's self force and then its entries); low half:
+// i, for centres without entries between.
+__global__ __launch_bounds__(256) void k_ext_fill(
+    int n, int M, const int* __restrict__ idx, const int* __restrict__ ctr,
+    const int* __restrict__ off, const int* __restrict__ start,
+    const int* __restrict__ rank, uint64_t* __restrict__ keys)
+{
+    int64_t const q = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (q >= (int64_t)M + n) return;
+    int const i = (int)(q - M);
+    int const b = q < M ? idx[q] : ctr[i];
+    keys[start[b] + rank[q]] = q < M
+        ? ((uint64_t)(2 * (uint32_t)q + 1) << 32)
+        : ((uint64_t)(2 * (uint32_t)off[i]) << 32) | (uint32_t)i;
+}
+
+// One wave per target puts its at most kExtSort contributions in order: the
+// rank of a key is the number of smaller ones.  src: q, or -(i + 1) for a
+// self force.
+__global__ __launch_bounds__(64) void k_ext_sort(
+    int nt, const int* __restrict__ start, const int* __restrict__ count,
+    const uint64_t* __restrict__ keys, int64_t* __restrict__ srcOff,
+    int* __restrict__ src)
+{
+    __shared__ uint64_t L[kExtSort];
+    int const b = blockIdx.x;
+    int const t0 = start[b], k = min(count[b], kExtSort);
+    for (int q = threadIdx.x; q < k; q += 64) L[q] = keys[t0 + q];
+    __syncthreads();
+    for (int q = threadIdx.x; q < k; q += 64)
+    {
+        uint64_t const key = L[q];
+        int r = 0;
+        for (int t = 0; t < k; ++t) r += L[t] < key;
+        uint32_t const hi = (uint32_t)(key >> 32);
+        src[t0 + r] = hi & 1 ? (int)(hi >> 1) : -(int)(uint32_t)key - 1;
+    }
+    if (threadIdx.x == 0)
+    {
+        srcOff[b] = t0;
+        if (b == nt - 1) srcOff[nt] = t0 + count[b];
+    }
+}
+
 // Exclusive scan helpers (block-level, then block offsets).
 __global__ void k_scan_block(const int* __restrict__ in, int* __restrict__ out,
                              int* __restrict__ blockSums, int n)
@@ -967,6 +1064,36 @@ hipError_t launch_list_stats(const int* count, int n, int* stats, int* host,
                              hipStream_t s)
 {
     k_list_stats<<<1, 1024, 0, s>>>(count, n, stats, host);
+    return hipGetLastError();
+}
+
+hipError_t launch_ext_entries(int n, int M, int ne, const int* idx,
+                              const int* elem, const double* dr, int* nbrJ,
+                              double4* geo, int* stats, hipStream_t s)
+{
+    int64_t const nb = ((int64_t)M + 255) / 256;
+    if (nb > 0)
+        k_ext_entries<<<(int)std::min<int64_t>(nb, 512), 256, 0, s>>>(
+            n, M, ne, idx, elem, dr, nbrJ, geo, stats);
+    return hipGetLastError();
+}
+
+hipError_t launch_ext_count(int n, int M, const int* idx, const int* ctr,
+                            int* count, int* rank, hipStream_t s)
+{
+    k_ext_count<<<(int)(((int64_t)M + n + 255) / 256), 256, 0, s>>>(
+        n, M, idx, ctr, count, rank);
+    return hipGetLastError();
+}
+
+hipError_t launch_ext_sort(int n, int M, int nt, const int* idx,
+                           const int* ctr, const int* off, const int* start,
+                           const int* count, const int* rank, uint64_t* keys,
+                           int64_t* srcOff, int* src, hipStream_t s)
+{
+    k_ext_fill<<<(int)(((int64_t)M + n + 255) / 256), 256, 0, s>>>(
+        n, M, idx, ctr, off, start, rank, keys);
+    k_ext_sort<<<nt, 64, 0, s>>>(nt, start, count, keys, srcOff, src);
     return hipGetLastError();
 }
 
