@@ -86,6 +86,22 @@ __device__ __forceinline__ void sincospi01(float x, float& s, float& c)
     c = __builtin_amdgcn_cosf(rev);
 }
 
+// sin and cos of pi r iw (FP32: half the scale as the revolutions, which
+// rounds as r iw / 2 does).
+__device__ __forceinline__ void sincospi_scaled(double r, double iw, double& s,
+                                                double& c)
+{
+    sincospi01(r * iw, s, c);
+}
+
+__device__ __forceinline__ void sincospi_scaled(float r, float iw, float& s,
+                                                float& c)
+{
+    float const rev = r * (0.5f * iw);
+    s = __builtin_amdgcn_sinf(rev);
+    c = __builtin_amdgcn_cosf(rev);
+}
+
 // 1/sqrt(x) for x > 0: hardware estimate refined by two Newton steps
 // y <- y (3 - x y^2) / 2 (each step squares the relative error).
 __device__ __forceinline__ double rsqrt_nr(double x)
@@ -228,6 +244,12 @@ __device__ __forceinline__ void cutoff_fdf_t(CutCfg const& c, R r, R& fc,
         dfc = x2 * ((R(60) - R(30) * x) * x - R(30)) * iw;
     }
 }
+
+// The cutoff configuration of a group: the model's one configuration as
+// literals where the model-specialised build defines it.
+#ifndef HDNNP_CUT
+#define HDNNP_CUT(cfg) (cfg)
+#endif
 
 // Launches KERNEL<CT, ...> for the cutoff types with specialised code and
 // KERNEL<-1, ...> (runtime switch) for the others.
@@ -476,11 +498,18 @@ __device__ __forceinline__ void cutoff_inside(CutCfg const& c, R r, R& fc,
     if (CT == CT_COS)
     {
         R const iw = (R)c.iw;
-        R x = (r - (R)c.rci) * iw;
-        x = fmin(fmax(x, R(0)), R(1));
         R sn, cs;
-        sincospi01(x, sn, cs);
-        fc = R(0.5) * (cs + R(1));
+        // No inner radius (known when the model's one cutoff is compiled in):
+        // x = r iw is in [0, 1] as it is.
+        if (__builtin_constant_p(c.rci) && c.rci == 0.0)
+            sincospi_scaled(r, iw, sn, cs);
+        else
+        {
+            R x = (r - (R)c.rci) * iw;
+            x = fmin(fmax(x, R(0)), R(1));
+            sincospi01(x, sn, cs);
+        }
+        fc = fma(R(0.5), cs, R(0.5));
         dfc = R(-0.5) * iw * (R)kPi * sn;
     }
     else if (CT == CT_POLY2)

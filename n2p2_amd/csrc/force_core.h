@@ -373,7 +373,7 @@ __device__ __forceinline__ void force_backward_body(ForceArgs const& a)
         // the neighbour's atomic number.
         int const cfg = ed.cfg0 + g.cfg;
         int const key = 2 * cfg + (weighted ? 1 : 0);
-        CutCfg const cc = T.cfg[cfg];
+        CutCfg const cc = HDNNP_CUT(T.cfg[cfg]);
         if (key != cfgCached)
         {
             // f_c and f_c'/r of every staged neighbour for this cutoff;

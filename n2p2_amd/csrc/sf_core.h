@@ -258,7 +258,7 @@ __device__ __forceinline__ void sf_forward_body(SFArgs const& a)
     for (int gi = ed.g0; gi < ed.g0 + ed.ng; ++gi)
     {
         GroupDesc const g = T.group[gi];
-        CutCfg const cc = T.cfg[ed.cfg0 + g.cfg];
+        CutCfg const cc = HDNNP_CUT(T.cfg[ed.cfg0 + g.cfg]);
         MemberDesc const* __restrict__ mem = T.member + g.mem0;
         int const nmem = g.nmem;
         bool const weighted = HDNNP_WEIGHTED && sf_weighted(g.type);
