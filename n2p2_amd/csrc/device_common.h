@@ -599,6 +599,25 @@ __device__ __forceinline__ double wave_sum_transposed(double (&v)[M])
     return t;
 }
 
+// Orders this wave's LDS accesses around a queue hand-off between lanes,
+// where the workgroup is one wave: a wave's LDS operations complete in
+// issue order, so a wavefront-scope fence (no wait, unlike the workgroup
+// barrier's fence) is enough and later LDS reads no longer wait for the
+// queue writes before them to complete.
+__device__ __forceinline__ void wave_lds_fence()
+{
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+}
+
+// Number of set bits of a 64-lane ballot below this lane (two mbcnt
+// instructions).
+__device__ __forceinline__ int lanes_below(uint64_t mask)
+{
+    return (int)__builtin_amdgcn_mbcnt_hi(
+        (unsigned)(mask >> 32),
+        __builtin_amdgcn_mbcnt_lo((unsigned)mask, 0u));
+}
+
 // Unordered pairs {j, k} of a group's neighbour blocks in diagonal order.
 // Same element (block of n at s0): pair p = c n + r is {r, (r + 1 + c) mod
 // n}, at circular distance 1 + c.  The (n - 1) / 2 full diagonals
@@ -675,23 +694,241 @@ __device__ __forceinline__ bool pair_in_range(V4 const& pj, V4 const& pk,
     return (pj.w < rc) & (pk.w < rc) & (wide | (d2 < rc2));
 }
 
-// Orders this wave's LDS accesses around a queue hand-off between lanes,
-// where the workgroup is one wave: a wave's LDS operations complete in
-// issue order, so a wavefront-scope fence (no wait, unlike the workgroup
-// barrier's fence) is enough and later LDS reads no longer wait for the
-// queue writes before them to complete.
-__device__ __forceinline__ void wave_lds_fence()
+// The model-specialised build says which angular types there are: 0 none of
+// the wide type, 1 only it, 2 both.
+#ifndef HDNNP_WIDE
+#define HDNNP_WIDE 2
+#endif
+
+// Keeps a value that was read from LDS with others in that one wide read: the
+// compiler otherwise splits it and reads the components that only a later
+// branch needs there, with 16-byte strides that collide in the banks.
+template <typename R>
+__device__ __forceinline__ void read_whole(R& x)
 {
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    asm volatile("" : "+v"(x));
 }
 
-// Number of set bits of a 64-lane ballot below this lane (two mbcnt
-// instructions).
-__device__ __forceinline__ int lanes_below(uint64_t mask)
+// Queue of a PairWalk: fewer than 64 entries when a step of 256 pairs starts,
+// and one that takes what is not queued.
+constexpr int kPairQueue = 64 + 256;
+constexpr int kPairQueueAlloc = kPairQueue + 4;
+
+typedef float Float4V __attribute__((ext_vector_type(4)));
+
+// Staged position and half its negative square, (x, y, z, -r^2 / 2), as the
+// pair search reads it; -1e30 in place of the square keeps the neighbour out
+// (r >= rc).  FP32 records give it as it is read, FP64 ones keep a float copy
+// M.
+constexpr float kOutside = -1e30f;
+
+__device__ __forceinline__ Float4V search_row(Vec4<float> const* P,
+                                              Float4V const*, float rc, int t)
 {
-    return (int)__builtin_amdgcn_mbcnt_hi(
-        (unsigned)(mask >> 32),
-        __builtin_amdgcn_mbcnt_lo((unsigned)mask, 0u));
+    Vec4<float> const p = P[t];
+    return Float4V{p.x, p.y, p.z, p.w < rc ? -0.5f * (p.w * p.w) : kOutside};
+}
+
+__device__ __forceinline__ Float4V search_row(Vec4<double> const*,
+                                              Float4V const* M, double, int t)
+{
+    return M[t];
+}
+
+__device__ __forceinline__ Float4V search_entry(double4 const& g)
+{
+    return Float4V{(float)g.x, (float)g.y, (float)g.z, kOutside};
+}
+
+// The pairs {j, k} of a group's neighbour blocks that can pass rij, rik < rc
+// and rjk < rc (narrow types), 64 at a time in diagonal order.
+//
+// Narrow: the search for rjk < rc is a matrix product.  With h = -r^2 / 2,
+// x_j x_k + y_j y_k + z_j z_k + h_j + h_k = -rjk^2 / 2, so five 4x4x1 MFMA
+// steps over 16 independent blocks give the distances of 16 blocks of 4 x 4
+// neighbours, 256 pairs, in 40 cycles of the matrix cores; the vector ALU
+// only compares (4) and appends the hits to the queue.  The blocks of 4 are
+// walked as DiagPairs walks single neighbours, and the four hits masks of a
+// step are recombined so that the 64 pairs of one append have 64 different j
+// and 64 different k (the force kernel's LDS adds collide on equal slots).
+// The distances are FP32 with an error below 2e-6 rc^2 (15 roundings of terms
+// up to 1.5 rc^2, h and, on the FP64 path, the rounded positions included),
+// so pairs up to 8e-6 rc^2 beyond are let through and the evaluation takes
+// f_c(rjk) = 0 for those (rij, rik < rc hold exactly: h).  One neighbour pair per lane and step (differences,
+// squares, index arithmetic and queue: 37 vector instructions per 64 pairs
+// instead of about 12) made the search 40% of the symmetry-function kernel.
+//
+// Wide: no distance to search; if every neighbour of the list is inside rc
+// (direct) the pairs go to the lanes as they come, else through the queue.
+template <typename R>
+struct PairWalk
+{
+    DiagPairs dp;         // neighbours (wide) or blocks of four (narrow)
+    Vec4<R> const* P;
+    Float4V const* M;
+    int* Q;
+    R rc;
+    float thr;
+    int s0, e0, l0, e1;   // first and last neighbour of each side
+    int base, qn, c, r;
+    bool wide, direct;
+
+    __device__ __forceinline__ PairWalk(bool wide_, bool allIn, bool same,
+                                        int a0, int na, int b0, int nb,
+                                        Vec4<R> const* P_, Float4V const* M_,
+                                        int* Q_, R rc_, R rc2)
+        : dp(same, a0, na, b0, nb), P(P_), M(M_), Q(Q_), rc(rc_),
+          thr(-0.5f * (1.0f + 8e-6f) * (float)rc2), base(0), qn(0), c(0),
+          r(0), wide(wide_), direct(wide_ && allIn)
+    {
+        s0 = dp.s0;
+        l0 = dp.l0;
+        e0 = s0 + dp.ns - 1;
+        e1 = l0 + dp.nl - 1;
+        if (!wide)
+        {
+            // Blocks of four: the same order with the diagonal (blocks with
+            // themselves) first.
+            int const nbs = (dp.ns + 3) >> 2, nbl = (dp.nl + 3) >> 2;
+            dp.d = nbs;
+            dp.nl = nbl;
+            dp.npairs = dp.npairs == 0 ? 0
+                      : same ? nbs * (nbs + 1) / 2 : nbs * nbl;
+            dp.q64 = nbs > 0 ? 16 / nbs : 0;
+            dp.r64 = 16 - dp.q64 * nbs;
+            dp.start(lane_id() >> 2, c, r);
+        }
+        else dp.start(lane_id(), c, r);
+    }
+
+    // 256 pairs of the narrow search.
+    __device__ __forceinline__ void search()
+    {
+        int const lane = lane_id(), j = lane & 3;
+        bool const valid = base + (lane >> 2) < dp.npairs;
+        int v = r + c;
+        if (v >= dp.nl) v -= dp.nl;
+        int const ja = s0 + 4 * r, kb = l0 + 4 * v + j;
+        // Beyond the end (also of the pairs): a neighbour in bounds, kept out.
+        Float4V A = search_row(P, M, rc, min(ja + j, e0));
+        Float4V B = search_row(P, M, rc, min(kb, e1));
+        if (ja + j > e0) A.w = kOutside;
+        if (kb > e1 || !valid) B.w = kOutside;
+        Float4V d = {0.0f, 0.0f, 0.0f, 0.0f};
+        d = __builtin_amdgcn_mfma_f32_4x4x1f32(A.x, B.x, d, 0, 0, 0);
+        d = __builtin_amdgcn_mfma_f32_4x4x1f32(A.y, B.y, d, 0, 0, 0);
+        d = __builtin_amdgcn_mfma_f32_4x4x1f32(A.z, B.z, d, 0, 0, 0);
+        d = __builtin_amdgcn_mfma_f32_4x4x1f32(A.w, 1.0f, d, 0, 0, 0);
+        d = __builtin_amdgcn_mfma_f32_4x4x1f32(1.0f, B.w, d, 0, 0, 0);
+        // d[i]: neighbour i of the first block, j of the second.  Rotated by
+        // j, so that d[s] is the pair (i = (j + s) mod 4, j).
+        bool const j1 = (j & 1) != 0, j2 = (j & 2) != 0;
+        float const t0 = j1 ? d[1] : d[0], t1 = j1 ? d[2] : d[1],
+                    t2 = j1 ? d[3] : d[2], t3 = j1 ? d[0] : d[3];
+        float p[4] = {j2 ? t2 : t0, j2 ? t3 : t1, j2 ? t0 : t2, j2 ? t1 : t3};
+        if (dp.same && base < dp.d)
+        {
+            // Blocks with themselves: i < j only, the s with j + s >= 4.
+            int const first = c == 0 ? 4 - j : 0;
+#pragma unroll
+            for (int s = 0; s < 4; ++s)
+                if (s < first) p[s] = kOutside;
+        }
+        int const code = ja | (kb << 16);
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+        {
+            uint64_t const hit = __ballot(p[s] > thr);
+            // The others write behind the queue.
+            int const at = __builtin_amdgcn_mbcnt_hi(
+                (uint32_t)(hit >> 32),
+                __builtin_amdgcn_mbcnt_lo((uint32_t)hit, qn));
+            Q[p[s] > thr ? at : kPairQueue] = code + ((j + s) & 3);
+            qn += __popcll(hit);
+        }
+        base += 16;
+        dp.advance(c, r);
+    }
+
+    // 64 pairs of a wide group with neighbours beyond rc.
+    __device__ __forceinline__ void filter()
+    {
+        bool const valid = base + lane_id() < dp.npairs;
+        int j, k;
+        dp.pair(c, r, j, k);
+        if (!valid) j = k = dp.s0;
+        bool const pass = valid & (P[j].w < rc) & (P[k].w < rc);
+        uint64_t const hit = __ballot(pass);
+        if (pass) Q[qn + lanes_below(hit)] = j | (k << 16);
+        qn += __popcll(hit);
+        base += 64;
+        dp.advance(c, r);
+    }
+
+    // Calls f(e, count) for the pairs in turn: e = j | k << 16 in the first
+    // `count` lanes.
+    template <typename F>
+    __device__ __forceinline__ void run(F const& f)
+    {
+        if (HDNNP_WIDE > 0 && direct)
+        {
+            for (; base < dp.npairs; base += 64)
+            {
+                int j, k;
+                dp.pair(c, r, j, k);
+                dp.advance(c, r);
+                f(j | (k << 16), min(64, dp.npairs - base));
+            }
+            return;
+        }
+        for (;;)
+        {
+            while (qn < 64 && base < dp.npairs)
+            {
+                if (HDNNP_WIDE == 0 || (HDNNP_WIDE == 2 && !wide)) search();
+                else filter();
+            }
+            int const count = min(64, qn);
+            if (count == 0) return;
+            wave_lds_fence();
+            qn -= count;
+            int const e = Q[qn + lane_id()];
+            wave_lds_fence();
+            f(e, count);
+        }
+    }
+};
+
+// Sums M per-lane values over the wave through LDS (M x 64 values at `s`,
+// 16-byte aligned): lane l adds M of the 64 values of member l / (64 / M),
+// in FP64, and a butterfly over the 64 / M lanes of a member follows.  Every
+// lane of member m's lanes returns its total; the order of the additions is
+// fixed.  About 35 vector instructions for 8 members; exchanging FP64 values
+// between lanes register by register takes about 250.
+template <int M, typename R>
+__device__ __forceinline__ double wave_sum_members(R const (&v)[M], R* s)
+{
+    static_assert(M == 4 || M == 8 || M == 16, "4, 8 or 16 members");
+    constexpr int kLanes = 64 / M, kVec = 16 / sizeof(R);
+    int const lane = lane_id();
+    wave_lds_fence();
+#pragma unroll
+    for (int m = 0; m < M; ++m) s[64 * m + lane] = v[m];
+    wave_lds_fence();
+    typedef R V __attribute__((ext_vector_type(16 / sizeof(R))));
+    V const* row = (V const*)(s + 64 * (lane / kLanes)) + lane % kLanes;
+    double t = 0.0;
+#pragma unroll
+    for (int q = 0; q < M / kVec; ++q)
+    {
+        V const x = row[q * kLanes];
+#pragma unroll
+        for (int u = 0; u < kVec; ++u) t += (double)x[u];
+    }
+    wave_lds_fence();
+#pragma unroll
+    for (int o = 1; o < kLanes; o <<= 1) t += __shfl_xor(t, o, kWave);
+    return t;
 }
 
 // Weight of staged neighbour t for the weighted SF types: the atomic number

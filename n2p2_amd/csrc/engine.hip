@@ -387,10 +387,12 @@ struct hdnnp_ctx
         T.genpow = 0;
         T.maxGroupMembers = 0;
         T.weighted = 0;
+        T.narrow = 0;
         for (auto const& g : flat.group)
         {
             T.maxGroupMembers = std::max(T.maxGroupMembers, g.nmem);
             if (sf_weighted(g.type)) T.weighted = 1;
+            if (!sf_radial(g.type) && g.type != 9) T.narrow = 1;
             if (!sf_radial(g.type))
                 for (int m = g.mem0; m < g.mem0 + g.nmem; ++m)
                     if (!flat.member[m].useint) T.genpow = 1;
@@ -960,7 +962,7 @@ void computeSF(hdnnp_ctx* c, bool raw)
     c->setDevice();
     int const cap = std::max(c->maxNeigh, 1);
     int const fp32 = (!raw && c->precision != HDNNP_PRECISION_FP64) ? 1 : 0;
-    if (sf_forward_lds_bytes(cap, fp32) > 65536
+    if (sf_list_lds_bytes(cap, fp32) > 65536
         || (c->T.ncgroup > 0 && sf_compact_lds_bytes(c->T, cap) > 65536))
         throw Error(HDNNP_E_CAPACITY,
                     "ERROR: Too many neighbours per atom for the symmetry-"
@@ -998,7 +1000,8 @@ void computeSF(hdnnp_ctx* c, bool raw)
     {
         void* params[] = {&a};
         hipCheck(hipModuleLaunchKernel(pk.sf, (unsigned)c->n, 1, 1, 64, 1, 1,
-                                       (unsigned)sf_forward_lds_bytes(cap,
+                                       (unsigned)sf_forward_lds_bytes(c->T,
+                                                                      cap,
                                                                       fp32),
                                        c->stream, params, nullptr),
                  "symmetry functions (specialised)");
@@ -1103,8 +1106,8 @@ void computeForces(hdnnp_ctx* c, int mode, bool wait = true)
     c->setDevice();
     int const cap = std::max(c->maxNeigh, 1);
     int const fp32 = c->precision != HDNNP_PRECISION_FP64 ? 1 : 0;
-    size_t const shm = force_backward_lds_bytes(cap, fp32);
-    if (shm > 65536
+    size_t const shm = force_backward_lds_bytes(c->T, cap, fp32);
+    if (force_list_lds_bytes(cap, fp32) > 65536
         || (c->T.ncgroup > 0 && force_compact_lds_bytes(c->T, cap) > 65536))
         throw Error(HDNNP_E_CAPACITY,
                     "ERROR: Too many neighbours per atom for the force "
@@ -3437,7 +3440,7 @@ int hdnnp_work_counts(hdnnp_ctx* c, int64_t* counts)
         requireNL(c);
         c->setDevice();
         int const cap = std::max(c->maxNeigh, 1);
-        if (sf_forward_lds_bytes(cap, 0) > 65536)
+        if (sf_list_lds_bytes(cap, 0) > 65536)
             throw Error(HDNNP_E_CAPACITY, "ERROR: Too many neighbours.\n");
         DBuf<unsigned long long> d;
         d.ensure(HDNNP_WORK_COUNTS);

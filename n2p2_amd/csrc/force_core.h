@@ -28,11 +28,11 @@
 //    current cutoff;
 //  * groups run one after another; a group's member parameters, with this
 //    atom's dE/dG weights, are held in scalar registers for the pair loop;
-//  * angular groups enumerate the unordered pairs {j, k} of their blocks in
-//    diagonal order (DiagPairs), test rij, rik < rc and rjk < rc (narrow) and
-//    push passing pairs into an LDS queue with a ballot prefix; whenever 64
-//    are queued every lane evaluates one triplet, so the work is divergence
-//    free and each triplet is evaluated once for both of its slots;
+//  * angular groups search the unordered pairs {j, k} of their blocks for
+//    those with rij, rik < rc and rjk < rc (narrow; PairWalk) and push them
+//    into an LDS queue; whenever 64 are queued every lane evaluates one
+//    triplet, so the work is divergence free and each triplet is evaluated
+//    once for both of its slots;
 //  * the member sum is contracted before the vector work.  With
 //    fg = exp(.) (1 + lambda cos)^(zeta-1) (SymGrpExpAngn.cpp:276-297) the
 //    reference's p1 (slot j), its mirror for slot k and p3 (:300-337) are
@@ -53,6 +53,9 @@
 //    order): the result does not depend on timing and repeats bit for bit.
 //    The diagonal pair order keeps the slots of a batch of 64 mostly
 //    distinct, so the adds rarely collide.
+// Bound by the LDS (six FP64 adds and four wide reads per triplet, 90% busy) in
+// FP32 and by vector instructions in FP64, where the search on the matrix
+// cores takes 196,608 water atoms from 5,230 to 5,090 us.
 #ifndef HDNNP_FORCE_CORE_H
 #define HDNNP_FORCE_CORE_H
 
@@ -79,7 +82,8 @@ struct BLds
                      // (FP64 on both paths): lanes on neighbouring slots
                      // hit neighbouring banks
     int cap;
-    int* QUEUE;      // kQueue passing pairs, j | k << 16
+    Float4V* M;      // FP64: float copy for the pair search
+    int* QUEUE;      // kPairQueue pairs, j | k << 16
 };
 
 template <typename R>
@@ -152,6 +156,7 @@ __device__ __forceinline__ void stage(ForceArgs const& a, BLds<R> const& S,
                     S.ACC[pos] = 0.0;
                     S.ACC[S.cap + pos] = 0.0;
                     S.ACC[2 * S.cap + pos] = 0.0;
+                    if (sizeof(R) == 8 && S.M) S.M[pos] = search_entry(g);
                 }
                 start[q] += __popcll(mask);
             }
@@ -194,13 +199,17 @@ __device__ __forceinline__ void lds_add(double* p, double v)
 }
 
 // One triplet {j, k} of angular group gi, all members: adds the slot-j and
-// slot-k contributions to the LDS accumulators.
+// slot-k contributions to the LDS accumulators.  Narrow: f_c(rjk) is taken as
+// 0 from rc on (rij, rik < rc).
 template <int CT, bool GENPOW, int MAXM, typename R>
 __device__ __forceinline__ void triplet_backward(
-    int gi, BLds<R> const& S, int j, int k, bool wide, CutCfg const& cc,
-    Members<R, MAXM> const& M, MParam<R> const* MP, int nmem)
+    int gi, BLds<R> const& S, int j, int k, bool wide, R rc2, CutCfg const& cc,
+    Members<R, MAXM> const& M, MParam<R> const* MP,
+    int nmem)
 {
-    Vec4<R> const pj = S.P[j], pk = S.P[k];
+    Vec4<R> pj = S.P[j], pk = S.P[k];
+    read_whole(pj.w);
+    read_whole(pk.w);
     Vec4<R> const qj = S.Q[j], qk = S.Q[k];
     R const rij = pj.w, rik = pk.w;
     R const fcij = qj.x, invj = qj.y, dfcij = qj.z;
@@ -219,6 +228,9 @@ __device__ __forceinline__ void triplet_backward(
         rjk = rjk2 * invjk;
         R fcjk, dfcjk;
         cutoff_inside<CT>(cc, rjk, fcjk, dfcjk);
+        bool const in = rjk2 < rc2;
+        fcjk = in ? fcjk : R(0);
+        dfcjk = in ? dfcjk : R(0);
         pfc = fij_ik * fcjk;
         r2sum = rij * rij + rik * rik + rjk2;
         pr1j = fcik * fcjk * dfcij;
@@ -340,17 +352,21 @@ __device__ __forceinline__ void force_backward_body(ForceArgs const& a)
     extern __shared__ __align__(16) double sm[];
     __shared__ int sStart[kMaxElements], sCnt[kMaxElements];
     __shared__ MParam<R> MP[kMaxMembers];
+    ModelTables const& T = a.T;
     int const cap = a.cap;
     BLds<R> S;
     S.P = (Vec4<R>*)sm;
     S.Q = S.P + cap;
     S.ACC = (double*)(S.Q + cap);
     S.cap = cap;
-    S.QUEUE = (int*)(S.ACC + 3 * cap);
+    constexpr bool kFloat = sizeof(R) == 4;
+    double* const end = S.ACC + 3 * cap + (cap & 1);    // 16-byte aligned
+    bool const copy = !kFloat && HDNNP_WIDE != 1 && T.narrow;
+    S.M = copy ? (Float4V*)end : nullptr;
+    S.QUEUE = copy ? (int*)(S.M + cap) : (int*)end;
 
     int const i = blockIdx.x;
     int const lane = threadIdx.x;
-    ModelTables const& T = a.T;
     int const ec = a.elem[i];
     ElemDesc const& ed = T.elem[ec];
     int const s0 = a.off[i];
@@ -365,6 +381,7 @@ __device__ __forceinline__ void force_backward_body(ForceArgs const& a)
     int pOff = kRecordGroups;
 
     int cfgCached = -1;
+    bool allIn = false;          // every neighbour inside the group's rc
     for (int gi = ed.g0; gi < ed.g0 + ed.ng; ++gi)
     {
         GroupDesc const g = T.group[gi];
@@ -380,10 +397,16 @@ __device__ __forceinline__ void force_backward_body(ForceArgs const& a)
             // weighted types: both times the neighbour's atomic number, so
             // every radial term carries Z_j and every triplet term Z_j Z_k
             // (SymGrpExpAngnWeighted.cpp:263-270).
+            bool out = false;
             for (int t = lane; t < n; t += 64)
             {
                 R f, df;
-                cutoff_fdf_t<CT>(cc, S.P[t].w, f, df);
+                R const r = S.P[t].w;
+                cutoff_fdf_t<CT>(cc, r, f, df);
+                bool const in = r < (R)g.rc;
+                out |= !in;
+                if (copy)
+                    S.M[t].w = in ? -0.5f * ((float)r * (float)r) : kOutside;
                 if (weighted)
                 {
                     R const z = (R)staged_weight(T, sStart, sCnt, t);
@@ -393,6 +416,7 @@ __device__ __forceinline__ void force_backward_body(ForceArgs const& a)
                 S.Q[t].x = f;
                 S.Q[t].z = df * S.Q[t].y;
             }
+            allIn = __ballot(out) == 0;
             cfgCached = key;
         }
         MemberDesc const* __restrict__ mem = T.member + g.mem0;
@@ -438,13 +462,16 @@ __device__ __forceinline__ void force_backward_body(ForceArgs const& a)
             continue;
         }
 
-        bool const wide = (g.type == 9);
+        bool const wide = HDNNP_WIDE == 2 ? g.type == 9 : HDNNP_WIDE == 1;
+        R const grc2 = (R)g.rc2;
         // Weighted type: all unordered pairs of the whole list.
-        DiagPairs const dp = weighted
-            ? DiagPairs(true, 0, n, 0, n)
-            : DiagPairs(g.e1 == g.e2, sStart[g.e1], sCnt[g.e1],
-                        sStart[g.e2], sCnt[g.e2]);
-        if (dp.npairs == 0)
+        PairWalk<R> walk(wide, allIn, weighted || g.e1 == g.e2,
+                         weighted ? 0 : uniform(sStart[g.e1]),
+                         weighted ? n : uniform(sCnt[g.e1]),
+                         weighted ? 0 : uniform(sStart[g.e2]),
+                         weighted ? n : uniform(sCnt[g.e2]), S.P, S.M,
+                         S.QUEUE, grc, grc2);
+        if (walk.dp.npairs == 0)
         {
             __syncthreads();
             continue;
@@ -452,7 +479,8 @@ __device__ __forceinline__ void force_backward_body(ForceArgs const& a)
         Members<R, MAXM> M;
         load_members(MP, nmem, M);
         int const nrec = rec && (gi - ed.g0) < kRecordGroups
-                       ? (int)rec[gi - ed.g0] : (int)kRecordMissing;
+                       ? uniform((int)rec[gi - ed.g0])
+                       : (int)kRecordMissing;
         if (nrec != (int)kRecordMissing)
         {
             // Replay the recorded pairs: the same triplets in the same lanes
@@ -466,45 +494,18 @@ __device__ __forceinline__ void force_backward_body(ForceArgs const& a)
                     next = rec[pOff + base + 64 + lane];
                 if (base + lane < nrec)
                     triplet_backward<CT, GENPOW, MAXM>(gi, S, e & 0xff,
-                                                       e >> 8, wide, cc, M,
-                                                       MP, nmem);
+                                                       e >> 8, wide, grc2, cc,
+                                                       M, MP, nmem);
             }
             pOff += nrec;
             __syncthreads();
             continue;
         }
-        R const grc2 = (R)g.rc2;
-        int qn = 0;
-        int pc, pr;
-        dp.start(lane, pc, pr);
-        for (int base = 0; base < dp.npairs; base += 64)
-        {
-            bool const valid = base + lane < dp.npairs;
-            int j, k;
-            dp.pair(pc, pr, j, k);
-            if (!valid) j = k = dp.s0;
-            dp.advance(pc, pr);
-            bool const pass = valid
-                & pair_in_range<R>(S.P[j], S.P[k], wide, grc, grc2);
-            uint64_t const mask = __ballot(pass);
-            if (pass) S.QUEUE[qn + lanes_below(mask)] = j | (k << 16);
-            qn += __popcll(mask);
-            wave_lds_fence();
-            if (qn >= 64)
-            {
-                int const e = S.QUEUE[qn - 64 + lane];
+        walk.run([&](int e, int count) {
+            if (lane < count)
                 triplet_backward<CT, GENPOW, MAXM>(gi, S, e & 0xffff, e >> 16,
-                                                   wide, cc, M, MP, nmem);
-                qn -= 64;
-                wave_lds_fence();
-            }
-        }
-        if (lane < qn)
-        {
-            int const e = S.QUEUE[lane];
-            triplet_backward<CT, GENPOW, MAXM>(gi, S, e & 0xffff, e >> 16,
-                                               wide, cc, M, MP, nmem);
-        }
+                                                   wide, grc2, cc, M, MP, nmem);
+        });
         __syncthreads();
     }
     // cself = -(sum of all slots), summed per lane in staged order and

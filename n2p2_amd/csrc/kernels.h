@@ -201,7 +201,10 @@ hipError_t launch_nl_partner(int n, const int* off, const int* cnt,
                              int* partner, int64_t nslots, hipStream_t s);
 
 hipError_t launch_sf_forward(SFArgs const& a, hipStream_t s);
-size_t sf_forward_lds_bytes(int cap, int fp32);
+// LDS of the kernels; the *_list_* sizes are their neighbour records and a
+// queue of kQueue pairs alone, the measure by which long lists are refused.
+size_t sf_forward_lds_bytes(ModelTables const& T, int cap, int fp32);
+size_t sf_list_lds_bytes(int cap, int fp32);
 // Work counters (10 x uint64, accumulated): see k_sf_count.
 hipError_t launch_sf_count(SFArgs const& a, unsigned long long* counters,
                            hipStream_t s);
@@ -215,7 +218,8 @@ hipError_t launch_sf_compact(SFArgs const& a, hipStream_t s);
 hipError_t launch_force_compact(ForceArgs const& a, hipStream_t s);
 size_t sf_compact_lds_bytes(ModelTables const& T, int cap);
 size_t force_compact_lds_bytes(ModelTables const& T, int cap);
-size_t force_backward_lds_bytes(int cap, int fp32);
+size_t force_backward_lds_bytes(ModelTables const& T, int cap, int fp32);
+size_t force_list_lds_bytes(int cap, int fp32);
 
 // Entries of atom i: [off[i], off[i] + cnt[i]).  order: the atoms sorted
 // by cell (processing order only).

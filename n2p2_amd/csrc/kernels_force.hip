@@ -126,20 +126,27 @@ void launch_bwd_r(ForceArgs const& a, size_t shm, hipStream_t s)
 
 }  // namespace
 
-size_t force_backward_lds_bytes(int cap, int fp32)
+size_t force_backward_lds_bytes(ModelTables const& T, int cap, int fp32)
 {
     size_t const r = fp32 ? sizeof(float) : sizeof(double);
     size_t b = 0;
     b += (size_t)cap * 8 * r;                     // P (4) and Q (4)
-    b += (size_t)cap * 3 * sizeof(double);        // ACC
-    b += (size_t)kQueue * sizeof(int);            // QUEUE
+    b += ((size_t)cap * 3 + (cap & 1)) * sizeof(double);    // ACC
+    if (!fp32 && T.narrow) b += (size_t)cap * 16;   // the search's float copy
+    b += (size_t)(T.narrow ? kPairQueueAlloc : kQueue) * sizeof(int);
     return b;
+}
+
+size_t force_list_lds_bytes(int cap, int fp32)
+{
+    return (size_t)cap * (8 * (fp32 ? sizeof(float) : sizeof(double))
+                          + 3 * sizeof(double)) + kQueue * sizeof(int);
 }
 
 hipError_t launch_force_backward(ForceArgs const& a, hipStream_t s)
 {
     if (a.n <= 0) return hipSuccess;
-    size_t const shm = force_backward_lds_bytes(a.cap, a.fp32);
+    size_t const shm = force_backward_lds_bytes(a.T, a.cap, a.fp32);
     if (a.fp32) launch_bwd_r<float>(a, shm, s);
     else launch_bwd_r<double>(a, shm, s);
     return hipGetLastError();

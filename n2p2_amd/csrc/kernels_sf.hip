@@ -5,6 +5,8 @@
 #include "sf_core.h"
 #include "kernels.h"
 
+#include <algorithm>
+
 namespace hdnnp {
 
 namespace {
@@ -181,7 +183,7 @@ __global__ void k_ew(ModelTables T, const double* __restrict__ G, int ldG,
 template <int MAXM, int CT, typename R>
 void launch_fwd(SFArgs const& a, hipStream_t s)
 {
-    size_t const shm = sf_forward_lds_bytes(a.cap, a.fp32);
+    size_t const shm = sf_forward_lds_bytes(a.T, a.cap, a.fp32);
     if (a.T.genpow)
         k_sf_forward<MAXM, CT, true, R><<<a.n, 64, shm, s>>>(a);
     else
@@ -200,10 +202,22 @@ void launch_fwd_r(SFArgs const& a, hipStream_t s)
 
 }  // namespace
 
-size_t sf_forward_lds_bytes(int cap, int fp32)
+size_t sf_forward_lds_bytes(ModelTables const& T, int cap, int fp32)
 {
+    // Records, FP64: the search's float copy, and the pair queue or the member
+    // sums of the largest chunk.
     size_t const r = fp32 ? sizeof(float) : sizeof(double);
-    return (size_t)cap * 6 * r + kQueue * sizeof(int);
+    size_t const even = (size_t)cap + (cap & 1);
+    int const maxm = T.maxGroupMembers <= 8 ? 8 : 16;
+    return even * (6 * r + (!fp32 && T.narrow ? 16 : 0))
+         + std::max<size_t>((T.narrow ? kPairQueueAlloc : kQueue)
+                            * sizeof(int), 64 * maxm * r);
+}
+
+size_t sf_list_lds_bytes(int cap, int fp32)
+{
+    return (size_t)cap * 6 * (fp32 ? sizeof(float) : sizeof(double))
+         + kQueue * sizeof(int);
 }
 
 hipError_t launch_sf_forward(SFArgs const& a, hipStream_t s)
@@ -218,7 +232,7 @@ hipError_t launch_sf_count(SFArgs const& a, unsigned long long* counters,
                            hipStream_t s)
 {
     if (a.n <= 0) return hipSuccess;
-    k_sf_count<<<a.n, 64, sf_forward_lds_bytes(a.cap, 0), s>>>(a, counters);
+    k_sf_count<<<a.n, 64, sf_list_lds_bytes(a.cap, 0), s>>>(a, counters);
     return hipGetLastError();
 }
 

@@ -367,7 +367,7 @@ __global__ __launch_bounds__(64) void k_train_u(TrainArgs A)
 template <int MAXM>
 void launch_train_u_m(TrainArgs const& A, hipStream_t s)
 {
-    size_t const shm = force_backward_lds_bytes(A.cap, 0);
+    size_t const shm = force_list_lds_bytes(A.cap, 0);
     if (A.T.genpow)
         HDNNP_CUTOFF_DISPATCH(A.T.cutType,
             (k_train_u<MAXM, kCT, true><<<A.n, 64, shm, s>>>(A)));

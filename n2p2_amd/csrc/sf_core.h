@@ -20,15 +20,20 @@
 //   2. groups run one after another; a group's member parameters are staged
 //      in LDS and the ones read per member held in scalar registers, its
 //      member sums live in registers;
-//   3. angular groups enumerate the unordered pairs of their blocks in
-//      diagonal order (DiagPairs), test
-//      rij, rik < rc and rjk < rc, and push passing pairs into an LDS queue
-//      with a ballot prefix; whenever 64 are queued every lane evaluates
-//      one, so the expensive triplet work runs without divergence;
+//   3. angular groups search the unordered pairs of their blocks for those
+//      with rij, rik < rc and rjk < rc (PairWalk) and push them into an LDS
+//      queue; whenever 64 are queued every lane evaluates one, so the
+//      expensive triplet work runs without divergence;
 //   4. inside a triplet the members are walked as (eta, rs) runs sharing one
 //      exponential and (eta, rs, lambda) runs sorted by zeta sharing one
 //      chain of powers of plambda (PowChain, bit-identical to pow_int);
-//   5. member sums are reduced with a fixed butterfly (deterministic).
+//   5. member sums are reduced through LDS in a fixed order (deterministic).
+// Bound by the issue of instructions (vector and scalar together; LDS and
+// memory are below 20%).  With the search on the matrix cores, the sums
+// through LDS and wide pairs straight to the lanes: 196,608 water atoms 2,190
+// -> 1,950 us in FP32 (1,716 us without the partner search beside it) and
+// 4,370 -> 3,970 us in FP64; 512 B/C/N structures (wide type only) 1,820 ->
+// 1,355 us.
 #ifndef HDNNP_SF_CORE_H
 #define HDNNP_SF_CORE_H
 
@@ -51,6 +56,7 @@ struct Stage
 {
     Vec4<R>* P;
     Vec2<R>* Q;      // null when only geometry is needed
+    Float4V* M = nullptr;   // FP64: float copy for the pair search
 };
 
 // Stages the atom's neighbours in LDS partitioned by element (stable ballot
@@ -117,6 +123,7 @@ __device__ void stage_by_element(SFArgs const& a, Stage<R> const& S, int s0,
                     p.w = (R)g.w;
                     S.P[pos] = p;
                     if (S.Q) S.Q[pos].y = R(1) / (R)g.w;
+                    if (S.M) S.M[pos] = search_entry(g);
                 }
                 start[q] += __popcll(mask);
             }
@@ -137,14 +144,17 @@ struct FwdMembers
 
 // One triplet, all members of the group: acc[m] += fg * plambda * pfc with
 // fg = exp(-eta sum r^2) plambda^(zeta - 1) (SymGrpExpAngn.cpp:276-297).
+// Narrow: f_c(rjk) is taken as 0 from rc on (rij, rik < rc).
 // ST: a staging record set with P (x, y, z, r) and Q (f_c, 1/r, ...).
 template <int MAXM, int CT, bool GENPOW, typename R, typename ST>
 __device__ __forceinline__ void triplet_forward(
-    int gi, ST const& S, int ja, int kb, bool wide, CutCfg const& cc,
-    FwdMembers<R, MAXM> const& M, MParam<R> const* MP, int nmem,
-    R (&acc)[MAXM])
+    int gi, ST const& S, int ja, int kb, bool wide, R rc2, CutCfg const& cc,
+    FwdMembers<R, MAXM> const& M, MParam<R> const* MP,
+    int nmem, R (&acc)[MAXM])
 {
-    Vec4<R> const pj = S.P[ja], pk = S.P[kb];
+    Vec4<R> pj = S.P[ja], pk = S.P[kb];
+    read_whole(pj.w);
+    read_whole(pk.w);
     auto const qj = S.Q[ja];
     auto const qk = S.Q[kb];
     R const rij = pj.w, rik = pk.w;
@@ -156,6 +166,7 @@ __device__ __forceinline__ void triplet_forward(
         rjk = rjk2 * rsqrt_nr(rjk2);
         R fcjk, dfcjk;
         cutoff_inside<CT>(cc, rjk, fcjk, dfcjk);
+        fcjk = rjk2 < rc2 ? fcjk : R(0);
         pfc = qj.x * qk.x * fcjk;
         r2sum = rij * rij + rik * rik + rjk2;
     }
@@ -227,15 +238,20 @@ __device__ __forceinline__ void sf_forward_body(SFArgs const& a)
     extern __shared__ __align__(16) double sm[];
     __shared__ int sStart[kMaxElements], sCnt[kMaxElements];
     __shared__ MParam<R> MP[kMaxMembers];
+    ModelTables const& T = a.T;
     int const cap = a.cap;
     Stage<R> S;
     S.P = (Vec4<R>*)sm;
     S.Q = (Vec2<R>*)(S.P + cap);
-    int* Q = (int*)(S.Q + cap);
+    // The pair queue, and between groups the member sums.  FP32: after an
+    // even number of 8-byte records.
+    constexpr bool kFloat = sizeof(R) == 4;
+    bool const copy = !kFloat && HDNNP_WIDE != 1 && T.narrow;
+    S.M = copy ? (Float4V*)(S.Q + cap) : nullptr;
+    int* Q = copy ? (int*)(S.M + cap) : (int*)(S.Q + (cap + (cap & 1)));
 
     int const i = blockIdx.x;
     int const lane = threadIdx.x;
-    ModelTables const& T = a.T;
     int const ec = a.elem[i];
     ElemDesc const& ed = T.elem[ec];
     int const s0 = a.off[i];
@@ -254,6 +270,7 @@ __device__ __forceinline__ void sf_forward_body(SFArgs const& a)
 
     double rcCached = -1.0;
     bool wCached = false;
+    bool allIn = false;          // every neighbour inside rcCached
     double* __restrict__ Gi = a.G + (size_t)i * a.ldG;
     for (int gi = ed.g0; gi < ed.g0 + ed.ng; ++gi)
     {
@@ -269,13 +286,20 @@ __device__ __forceinline__ void sf_forward_body(SFArgs const& a)
             // radial terms carry Z_j and triplet products Z_j Z_k
             // (SymGrpExpRadWeighted.cpp:200-207,
             // SymGrpExpAngnWeighted.cpp:263-270).
+            bool out = false;
             for (int t = lane; t < n; t += 64)
             {
                 R f, df;
-                cutoff_fdf_t<CT>(cc, S.P[t].w, f, df);
+                R const r = S.P[t].w;
+                cutoff_fdf_t<CT>(cc, r, f, df);
                 if (weighted) f *= (R)staged_weight(T, sStart, sCnt, t);
                 S.Q[t].x = f;
+                bool const in = r < (R)g.rc;
+                out |= !in;
+                if (copy)
+                    S.M[t].w = in ? -0.5f * ((float)r * (float)r) : kOutside;
             }
+            allIn = __ballot(out) == 0;
             rcCached = g.rc;
             wCached = weighted;
         }
@@ -307,13 +331,15 @@ __device__ __forceinline__ void sf_forward_body(SFArgs const& a)
         }
         else
         {
-            bool const wide = (g.type == 9);
+            bool const wide = HDNNP_WIDE == 2 ? g.type == 9 : HDNNP_WIDE == 1;
             // Weighted type: all unordered pairs of the whole list.
-            DiagPairs const dp = weighted
-                ? DiagPairs(true, 0, n, 0, n)
-                : DiagPairs(g.e1 == g.e2, sStart[g.e1], sCnt[g.e1],
-                            sStart[g.e2], sCnt[g.e2]);
             R const grc = (R)g.rc, grc2 = (R)g.rc2;
+            PairWalk<R> walk(wide, allIn, weighted || g.e1 == g.e2,
+                             weighted ? 0 : uniform(sStart[g.e1]),
+                             weighted ? n : uniform(sCnt[g.e1]),
+                             weighted ? 0 : uniform(sStart[g.e2]),
+                             weighted ? n : uniform(sCnt[g.e2]), S.P, S.M, Q,
+                             grc, grc2);
             FwdMembers<R, MAXM> M;
 #pragma unroll
             for (int m = 0; m < MAXM; ++m)
@@ -322,74 +348,34 @@ __device__ __forceinline__ void sf_forward_body(SFArgs const& a)
                 M.lam[m] = uniform_r(p.lambda);
                 M.code[m] = uniform(p.flags);
             }
-            // Passing pairs of this group go to the record while they fit,
-            // in the order and lane positions the force kernel would meet
-            // them (staged indices j | k << 8).
+            // The pairs of this group go to the record while they fit, in
+            // the order and lane positions the force kernel's own walk would
+            // meet them (staged indices j | k << 8).
             bool keep = record && (gi - ed.g0) < kRecordGroups;
             int nrec = 0;
-            int qn = 0;
-            int pc = 0, pr = 0;
-            dp.start(lane, pc, pr);
-            for (int base = 0; base < dp.npairs; base += 64)
-            {
-                bool const valid = base + lane < dp.npairs;
-                int ja, kb;
-                dp.pair(pc, pr, ja, kb);
-                if (!valid) ja = kb = dp.s0;
-                dp.advance(pc, pr);
-                // Invalid lanes test (s0, s0), in bounds: no divergent
-                // branch around the LDS reads.
-                bool const pass = valid
-                    & pair_in_range<R>(S.P[ja], S.P[kb], wide, grc, grc2);
-                uint64_t const mask = __ballot(pass);
-                if (pass) Q[qn + lanes_below(mask)] = ja | (kb << 16);
-                qn += __popcll(mask);
-                wave_lds_fence();
-                if (qn >= 64)
-                {
-                    int const e = Q[qn - 64 + lane];
+            walk.run([&](int e, int count) {
+                if (lane < count)
                     triplet_forward<MAXM, CT, GENPOW>(gi, S, e & 0xffff,
-                                                      e >> 16, wide, cc, M, MP,
-                                                      nmem, acc);
-                    if (keep && pOff + nrec + 64 <= a.pcap)
-                    {
-                        rec[pOff + nrec + lane] = (unsigned short)(
-                            (e & 0xff) | ((e >> 16) << 8));
-                        nrec += 64;
-                    }
-                    else keep = false;
-                    qn -= 64;
-                    wave_lds_fence();
-                }
-            }
-            if (lane < qn)
-            {
-                int const e = Q[lane];
-                triplet_forward<MAXM, CT, GENPOW>(gi, S, e & 0xffff, e >> 16,
-                                                  wide, cc, M, MP, nmem, acc);
-            }
-            if (keep && pOff + nrec + qn <= a.pcap)
-            {
-                if (lane < qn)
-                {
-                    int const e = Q[lane];
+                                                      e >> 16, wide, grc2, cc,
+                                                      M, MP, nmem, acc);
+                keep = keep && pOff + nrec + count <= a.pcap;
+                if (keep && lane < count)
                     rec[pOff + nrec + lane] = (unsigned short)(
                         (e & 0xff) | ((e >> 16) << 8));
-                }
-                nrec += qn;
+                nrec += count;
+            });
+            if (keep)
+            {
                 if (lane == 0) rec[gi - ed.g0] = (unsigned short)nrec;
                 pOff += nrec;
             }
         }
-        // Member totals by the transposing butterfly: member m ends in the
-        // lanes (m << (6 - log2 MAXM)) + t; the first of them writes it.
-        double dv[MAXM];
-#pragma unroll
-        for (int m = 0; m < MAXM; ++m) dv[m] = (double)acc[m];
-        double const v = wave_sum_transposed<MAXM>(dv);
-        constexpr int kSh = MAXM == 4 ? 4 : MAXM == 8 ? 3 : 2;   // 6 - log2
-        int const m = lane >> kSh;
-        if ((lane & ((1 << kSh) - 1)) == 0 && m < nmem)
+        // Member m's total ends in lanes m 64 / MAXM and up; the first of them
+        // writes it.
+        double const v = wave_sum_members(acc, (R*)Q);
+        constexpr int kLanes = 64 / MAXM;
+        int const m = lane / kLanes;
+        if (lane % kLanes == 0 && m < nmem)
         {
             MemberDesc const& md = mem[m];
             double const raw = sf_radial(g.type) ? v : v * md.gfac;

@@ -289,8 +289,18 @@ std::string cut_source(Model::Flat const& F)
     return o.str();
 }
 
+// HDNNP_WIDE of a model's angular groups.
+int plan_wide(Model::Flat const& F)
+{
+    bool wide = false, narrow = false;
+    for (GroupDesc const& g : F.group)
+        if (!sf_radial(g.type)) (g.type == 9 ? wide : narrow) = true;
+    return wide && narrow ? 2 : wide ? 1 : 0;
+}
+
 std::string full_source(std::string const& plan, std::string const& cut,
-                        ModelTables const& T, int fp32, PlanTuning const& tune)
+                        int wide, ModelTables const& T, int fp32,
+                        PlanTuning const& tune)
 {
     std::ostringstream o;
     char const* R = fp32 ? "float" : "double";
@@ -299,6 +309,7 @@ std::string full_source(std::string const& plan, std::string const& cut,
     // Models without weighted groups leave the weighted code out.
     o << "#define HDNNP_PLAN 1\n"
       << "#define HDNNP_WEIGHTED " << (T.weighted ? 1 : 0) << "\n"
+      << "#define HDNNP_WIDE " << wide << "\n"
       << "#include \"device_common.h\"\n"
       << "#include \"kernel_args.h\"\n"
       << "namespace hdnnp {\nnamespace {\n" << plan << "}\n}\n" << cut
@@ -449,8 +460,8 @@ bool plan_enabled_by_default()
 PlanKernels plan_kernels(Model::Flat const& F, ModelTables const& T,
                          int fp32, int device, PlanTuning const& tune)
 {
-    std::string const src = full_source(plan_source(F), cut_source(F), T,
-                                        fp32, tune);
+    std::string const src = full_source(plan_source(F), cut_source(F),
+                                        plan_wide(F), T, fp32, tune);
     // Keyed by the full source (a few tens of KB): no collisions.
     std::string const key = std::to_string(device) + ":" + src;
     std::lock_guard<std::mutex> lock(g_mutex);

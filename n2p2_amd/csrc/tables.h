@@ -203,6 +203,7 @@ struct ModelTables
     int genpow;           // some angular member has a non-integer zeta
     int maxGroupMembers;  // largest group chunk
     int weighted;         // some group is of a weighted type (12, 13)
+    int narrow;           // some angular group tests rjk (3, 13)
     double maxCutoff;
     double zw[kMaxElements];      // atomic number per element (weights of
                                   // the weighted types)
