@@ -823,8 +823,15 @@ void buildNeighborList(hdnnp_ctx* c, double rc)
     // Cell-per-workgroup kernels when at most 64 neighbour cells are searched
     // and every cell's candidates fit their LDS; the per-atom kernels
     // otherwise.  Both produce the same list.
-    bool cellKernels = (2 * p.m[0] + 1) * (2 * p.m[1] + 1) * (2 * p.m[2] + 1)
-                     <= 64;
+    int const ncand = (2 * p.m[0] + 1) * (2 * p.m[1] + 1) * (2 * p.m[2] + 1);
+    bool cellKernels = ncand <= 64;
+    // The larger staging at once where cells of 15% more than the mean need it.
+    int cand = 1.15 * ncand * n / ncell > kCellCand ? kCellCandMax : kCellCand;
+    // After a staging overflow of `need` candidates.
+    auto overflow = [&](int need) {
+        if (cand < need && need <= kCellCandMax) cand = kCellCandMax;
+        else cellKernels = false;
+    };
     int hstat[4] = {0, 0, 0, 0};
     bool built = false;
     if (cellKernels && c->slab > 0 && c->slabAtoms == n)
@@ -838,21 +845,22 @@ void buildNeighborList(hdnnp_ctx* c, double rc)
                                      c->dCellCount.p, c->dCellAtoms.p,
                                      c->dCount.p, c->dStats.p, c->dOff.p,
                                      c->slab, c->dKeys.p, c->dNbrJ.p,
-                                     c->dGeo.p, s), "nl fill");
+                                     c->dGeo.p, cand, s), "nl fill");
         readStats(c, c->dCount.p, n, hstat);
-        if (hstat[2] > 0) cellKernels = false;    // staging overflow
+        if (hstat[2] > 0) overflow(hstat[2]);
         else if (hstat[3] == 0) built = true;
     }
     int maxc = hstat[0];
     if (!built)
     {
-        for (int attempt = 0; attempt < 2; ++attempt)
+        for (;;)
         {
             if (cellKernels)
                 hipCheck(launch_nl_count_cell(p, ncell, c->dR.p,
                                               c->dCellStart.p, c->dCellCount.p,
                                               c->dCellAtoms.p, c->dCount.p,
-                                              c->dStats.p, s), "nl count");
+                                              c->dStats.p, cand, s),
+                         "nl count");
             else
                 hipCheck(launch_nl_count(p, c->dR.p, c->dElemAtom.p,
                                          c->dCellOfAtom.p, c->dCellStart.p,
@@ -861,7 +869,7 @@ void buildNeighborList(hdnnp_ctx* c, double rc)
                          "nl count");
             readStats(c, c->dCount.p, n, hstat);
             if (!(cellKernels && hstat[2] > 0)) break;
-            cellKernels = false;     // a cell overflowed the staging: redo
+            overflow(hstat[2]);      // redo
         }
         maxc = hstat[0];
         if (cellKernels)
@@ -878,7 +886,7 @@ void buildNeighborList(hdnnp_ctx* c, double rc)
                                          c->dCellCount.p, c->dCellAtoms.p,
                                          c->dCount.p, c->dStats.p, c->dOff.p,
                                          c->slab, c->dKeys.p, c->dNbrJ.p,
-                                         c->dGeo.p, s), "nl fill");
+                                         c->dGeo.p, cand, s), "nl fill");
         }
         else
         {

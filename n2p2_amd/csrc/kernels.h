@@ -43,12 +43,15 @@ hipError_t launch_nl_fill(NLParams const& p, const double* r, const int* elem,
                           uint64_t* keys, int* nbrJ, double4* geo,
                           hipStream_t s);
 // Cell-per-workgroup variants (at most 64 neighbour cells searched):
-// stats[2] receives the largest staged candidate count when a cell exceeds
-// the kernel's LDS capacity (the caller then uses the per-atom kernels).
+// stats[2] receives the largest candidate count of a cell when one exceeds the
+// kernel's staging (the caller then takes the larger form or the per-atom
+// kernels).  cand picks the smallest of the two forms that holds it.
+constexpr int kCellCand = 1024;
+constexpr int kCellCandMax = 2048;
 hipError_t launch_nl_count_cell(NLParams const& p, int ncell, const double* r,
                                 const int* cellStart, const int* cellCount,
                                 const int* cellAtoms, int* count, int* stats,
-                                hipStream_t s);
+                                int cand, hipStream_t s);
 // Writes atom i's entries from off[i] on, at most limit of them; count[i]
 // receives the true count, stats[3] = 1 if a count exceeds limit (the
 // largest count: launch_list_stats over count).
@@ -56,7 +59,8 @@ hipError_t launch_nl_fill_cell(NLParams const& p, int ncell, const double* r,
                                const int* cellStart, const int* cellCount,
                                const int* cellAtoms, int* count, int* stats,
                                const int* off, int limit, uint64_t* keys,
-                               int* nbrJ, double4* geo, hipStream_t s);
+                               int* nbrJ, double4* geo, int cand,
+                               hipStream_t s);
 // Cell of one structure of a batch.  The host sets everything but the
 // atoms' fractional extent fmin/fmax, which launch_batch_extent fills.
 struct BatchCell

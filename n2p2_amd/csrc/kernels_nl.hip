@@ -270,22 +270,32 @@ __global__ __launch_bounds__(64) void k_nl(
 
 // Cell kernels: one workgroup of four waves per cell.  The atoms of the
 // cell's (2m+1)^3 neighbour cells (m = 1 when cells are at least rc wide)
-// are staged once in LDS with their image vectors; each wave then takes one
-// atom of the cell at a time and tests all staged candidates, 64 per step.
-// MODE 0 counts hits.  MODE 1 first sorts the staged candidates by
-// (j, image), the reference's loop order, so that the ballot compaction of
-// an atom's hits is already in list order and they are written directly.
+// are staged once in LDS as keys and FP32 positions relative to the cell's
+// first atom; each wave then takes one atom of the cell at a time and tests
+// all staged candidates, 64 per step.  MODE 0 counts hits.  MODE 1 first sorts
+// the candidates by (j, image), the reference's loop order, so that an atom's
+// hits come in list order and are written directly.
+// The FP32 test lets through whatever the rounding of the positions could
+// hide (thr below); what passes, about one candidate in seven, goes through a
+// queue per wave to the exact FP64 test in the reference's operation order,
+// 64 at a time and in order.
 // The host uses these kernels when at most 64 neighbour cells are searched
-// and falls back to k_nl when a cell has more than kCellCand candidates
-// (stats[2]).  MODE 1 writes atom i's entries from off[i] on, at most
-// limit of them (a fixed slot range per atom), stores the true count in
+// and falls back to k_nl when a cell has more candidates than the larger
+// staging holds (stats[2]).  MODE 1 writes atom i's entries from off[i] on, at
+// most limit of them (a fixed slot range per atom), stores the true count in
 // count[i] and sets stats[3] when a count exceeds limit (the host then
 // rebuilds with a larger range); the largest count comes from a reduction
 // over count[] afterwards (launch_list_stats).
-constexpr int kCellCand = 1024;
+// Bound by vector instructions.  With the FP64 image arithmetic for every
+// candidate, 32 KiB of FP64 staging and a workgroup barrier after each of the
+// sort's stages, the lists of 196,608 water atoms (28.7 atoms and 774
+// candidates per cell) took 643 us, now 395 us.  CAND: 1024 candidates (23 KiB
+// of LDS, seven workgroups per CU), or 2048 (43 KiB) for the wider cells of
+// lists with a skin, which the per-atom kernels built in 336 us for 24,576
+// atoms (rc 7.35 A, 1,296 candidates), now 150 us.
 constexpr int kCellWaves = 4;
 
-template <int MODE>
+template <int MODE, int CAND>
 __global__ __launch_bounds__(256) void k_nl_cell(
     NLParams p, const double* __restrict__ r,
     const int* __restrict__ cellStart, const int* __restrict__ cellCount,
@@ -294,10 +304,10 @@ __global__ __launch_bounds__(256) void k_nl_cell(
     uint64_t* __restrict__ keysOut, int* __restrict__ nbrJ,
     double4* __restrict__ geo)
 {
-    __shared__ double cX[kCellCand], cY[kCellCand], cZ[kCellCand];
-    // MODE 0: (j << 21 | image).  MODE 1: (j << 31 | image << 10 | t), t the
-    // staging slot, sorted.
-    __shared__ uint64_t cKey[kCellCand];
+    __shared__ float cX[CAND], cY[CAND], cZ[CAND];
+    __shared__ uint64_t cKey[CAND];              // make_key, MODE 1: sorted
+    __shared__ int queue[kCellWaves][128];
+    __shared__ int sFar;                         // largest |coordinate| (bits)
     __shared__ int sStart[64], sCnt[64], sPre[64], sImg[64];
     __shared__ int sTotal;
     // Cells in XCD-aware order: each XCD takes a contiguous range of cells,
@@ -351,10 +361,11 @@ __global__ __launch_bounds__(256) void k_nl_cell(
         sPre[tid] = pre - cnt;
         sImg[tid] = img;
         if (tid == 63) sTotal = pre;
+        if (tid == 0) sFar = 0;
     }
     __syncthreads();
     int const total = sTotal;
-    if (total > kCellCand)
+    if (total > CAND)
     {
         if (tid == 0) atomicMax(&stats[2], total);
         return;
@@ -377,18 +388,13 @@ __global__ __launch_bounds__(256) void k_nl_cell(
         }
         while (lo > 0 && (sCnt[lo] == 0 || sPre[lo] + sCnt[lo] <= t)) --lo;
         int const j = cellAtoms[sStart[lo] + (t - sPre[lo])];
-        cX[t] = r[3 * (size_t)j];
-        cY[t] = r[3 * (size_t)j + 1];
-        cZ[t] = r[3 * (size_t)j + 2];
-        uint64_t const img = (uint64_t)sImg[lo];
-        cKey[t] = MODE == 1
-                ? ((uint64_t)(uint32_t)j << 31) | (img << 10) | (uint64_t)t
-                : ((uint64_t)(uint32_t)j << 21) | img;
+        cKey[t] = ((uint64_t)(uint32_t)j << 21) | (uint64_t)sImg[lo];
     }
     __syncthreads();
     if (MODE == 1)
     {
-        // bitonic sort of cKey[0, P)
+        // Bitonic sort of cKey[0, P).  Exchanges below 64 stay within the 64
+        // keys of a wave's pass, which needs no workgroup barrier.
         for (int k = 2; k <= P; k <<= 1)
         {
             for (int jj = k >> 1; jj > 0; jj >>= 1)
@@ -407,94 +413,107 @@ __global__ __launch_bounds__(256) void k_nl_cell(
                         }
                     }
                 }
-                __syncthreads();
-            }
-        }
-    }
-    if (MODE == 1)
-    {
-        // Candidate coordinates into sorted order (slot u holds the
-        // candidate of the u-th key), so that the scan below reads them
-        // with consecutive, conflict-free LDS accesses.
-        constexpr int kPer = kCellCand / 256;
-        double px[kPer], py[kPer], pz[kPer];
-#pragma unroll
-        for (int q = 0; q < kPer; ++q)
-        {
-            int const u = tid + 256 * q;
-            if (u < total)
-            {
-                int const t = (int)(cKey[u] & 1023);
-                px[q] = cX[t];
-                py[q] = cY[t];
-                pz[q] = cZ[t];
+                // The next exchange: jj / 2, or k from jj = 1.
+                if (jj >= 64 || (jj == 1 && k >= 64))
+                    __syncthreads();
+                else wave_lds_fence();
             }
         }
         __syncthreads();
-#pragma unroll
-        for (int q = 0; q < kPer; ++q)
-        {
-            int const u = tid + 256 * q;
-            if (u < total)
-            {
-                cX[u] = px[q];
-                cY[u] = py[q];
-                cZ[u] = pz[q];
-            }
-        }
     }
-    __syncthreads();
     int const a0 = cellStart[cell];
+    double org[3];
+    {
+        int const i0 = cellAtoms[a0];
+        for (int k = 0; k < 3; ++k) org[k] = r[3 * (size_t)i0 + k];
+    }
+    float far = 0.0f;
+    for (int t = tid; t < total; t += 256)
+    {
+        int j, b0, b1, b2;
+        split_key(cKey[t], j, b0, b1, b2);
+        double const rj[3] = {r[3 * (size_t)j], r[3 * (size_t)j + 1],
+                              r[3 * (size_t)j + 2]};
+        double dr[3];
+        image_dr(p, org, rj, b0, b1, b2, dr);
+        float const x = (float)dr[0], y = (float)dr[1], z = (float)dr[2];
+        cX[t] = x;
+        cY[t] = y;
+        cZ[t] = z;
+        far = fmaxf(far, fmaxf(fabsf(x), fmaxf(fabsf(y), fabsf(z))));
+    }
+    for (int o = 32; o > 0; o >>= 1) far = fmaxf(far, __shfl_xor(far, o));
+    if (lane == 0) atomicMax(&sFar, __float_as_int(far));
+    __syncthreads();
+    // FP32 test.  A coordinate is off by 2^-24 far and a difference of two by
+    // e = 2^-23 far (and its own rounding), so d^2 near rc^2 is off by at most
+    // 2 sqrt(3) rc e + 3 e^2 and a few 2^-24 rc^2: wider margins than that.
+    float const frc = (float)sqrt(p.rc2);
+    float const err = 1.1920929e-7f * __int_as_float(sFar);
+    float const thr = frc * frc * (1.0f + 4e-6f) + (8.0f * frc + 4.0f * err)
+                                                   * err;
+    int* const Q = queue[w];
     for (int a = w; a < nAt; a += kCellWaves)
     {
         int const i = cellAtoms[a0 + a];
         double const ri[3] = {r[3 * (size_t)i], r[3 * (size_t)i + 1],
                               r[3 * (size_t)i + 2]};
+        // As the candidates (org - r_i), so that the origin cancels.
+        float const x = (float)(org[0] - ri[0]), y = (float)(org[1] - ri[1]),
+                    z = (float)(org[2] - ri[2]);
+        uint64_t const self = make_key(i, 0, 0, 0);
         int const o = MODE == 1 ? off[i] : 0;
-        int hits = 0;
-        for (int u0 = 0; u0 < total; u0 += 64)
-        {
-            int const u = u0 + lane;
+        int hits = 0, qn = 0;
+        // The first `c` queued candidates, exactly.
+        auto flush = [&](int c) {
             bool hit = false;
-            int j = 0, img = 0, t = 0;
+            uint64_t key = 0;
+            int j = 0;
             double dr[3] = {0.0, 0.0, 0.0};
-            if (u < total)
+            if (lane < c)
             {
-                uint64_t const ck = cKey[u];
-                if (MODE == 1)
-                {
-                    j = (int)(ck >> 31);
-                    img = (int)((ck >> 10) & 0x1fffff);
-                    t = u;   // coordinates are in sorted order
-                }
-                else
-                {
-                    j = (int)(ck >> 21);
-                    img = (int)(ck & 0x1fffff);
-                    t = u;
-                }
-                if (!(j == i && img == zeroImg))
-                {
-                    int const b0 = ((img >> 14) & 127) - kBias;
-                    int const b1 = ((img >> 7) & 127) - kBias;
-                    int const b2 = (img & 127) - kBias;
-                    double const rj[3] = {cX[t], cY[t], cZ[t]};
-                    image_dr(p, ri, rj, b0, b1, b2, dr);
-                    hit = norm2_pinned(dr) <= p.rc2;
-                }
+                int b0, b1, b2;
+                key = cKey[Q[lane]];
+                split_key(key, j, b0, b1, b2);
+                double const rj[3] = {r[3 * (size_t)j], r[3 * (size_t)j + 1],
+                                      r[3 * (size_t)j + 2]};
+                image_dr(p, ri, rj, b0, b1, b2, dr);
+                hit = key != self && norm2_pinned(dr) <= p.rc2;
             }
             uint64_t const mask = __ballot(hit);
             int const h = hits + lanes_below(mask);
             if (MODE == 1 && hit && h < limit)
             {
                 int const q = o + h;
-                keysOut[q] = ((uint64_t)(uint32_t)j << 21) | (uint64_t)img;
+                keysOut[q] = key;
                 nbrJ[q] = j;
                 geo[q] = make_double4(dr[0], dr[1], dr[2],
                                       sqrt(norm2_pinned(dr)));
             }
             hits += __popcll(mask);
+        };
+        for (int u0 = 0; u0 < total; u0 += 64)
+        {
+            int const u = min(u0 + lane, total - 1);
+            float const dx = cX[u] - x, dy = cY[u] - y, dz = cZ[u] - z;
+            bool const in = (u0 + lane < total)
+                          & (dx * dx + dy * dy + dz * dz <= thr);
+            uint64_t const mask = __ballot(in);
+            if (in) Q[qn + lanes_below(mask)] = u;
+            qn += __popcll(mask);
+            wave_lds_fence();
+            if (qn >= 64)
+            {
+                flush(64);
+                int const rest = Q[64 + lane];
+                wave_lds_fence();
+                Q[lane] = rest;
+                wave_lds_fence();
+                qn -= 64;
+            }
         }
+        flush(qn);
+        wave_lds_fence();
         if (lane == 0)
         {
             count[i] = hits;
@@ -1141,12 +1160,13 @@ hipError_t launch_nl_fill(NLParams const& p, const double* r, const int* elem,
 hipError_t launch_nl_count_cell(NLParams const& p, int ncell, const double* r,
                                 const int* cellStart, const int* cellCount,
                                 const int* cellAtoms, int* count, int* stats,
-                                hipStream_t s)
+                                int cand, hipStream_t s)
 {
     if (ncell <= 0) return hipSuccess;
-    k_nl_cell<0><<<ncell, 256, 0, s>>>(p, r, cellStart, cellCount, cellAtoms,
-                                       count, stats, nullptr, 0, nullptr,
-                                       nullptr, nullptr);
+    auto const k = cand > kCellCand ? k_nl_cell<0, kCellCandMax>
+                                    : k_nl_cell<0, kCellCand>;
+    k<<<ncell, 256, 0, s>>>(p, r, cellStart, cellCount, cellAtoms, count,
+                            stats, nullptr, 0, nullptr, nullptr, nullptr);
     return hipGetLastError();
 }
 
@@ -1154,12 +1174,14 @@ hipError_t launch_nl_fill_cell(NLParams const& p, int ncell, const double* r,
                                const int* cellStart, const int* cellCount,
                                const int* cellAtoms, int* count, int* stats,
                                const int* off, int limit, uint64_t* keys,
-                               int* nbrJ, double4* geo, hipStream_t s)
+                               int* nbrJ, double4* geo, int cand,
+                               hipStream_t s)
 {
     if (ncell <= 0) return hipSuccess;
-    k_nl_cell<1><<<ncell, 256, 0, s>>>(p, r, cellStart, cellCount, cellAtoms,
-                                       count, stats, off, limit, keys, nbrJ,
-                                       geo);
+    auto const k = cand > kCellCand ? k_nl_cell<1, kCellCandMax>
+                                    : k_nl_cell<1, kCellCand>;
+    k<<<ncell, 256, 0, s>>>(p, r, cellStart, cellCount, cellAtoms, count,
+                            stats, off, limit, keys, nbrJ, geo);
     return hipGetLastError();
 }
 
