@@ -464,18 +464,6 @@ __device__ __forceinline__ void force_backward_body(ForceArgs const& a)
 
         bool const wide = HDNNP_WIDE == 2 ? g.type == 9 : HDNNP_WIDE == 1;
         R const grc2 = (R)g.rc2;
-        // Weighted type: all unordered pairs of the whole list.
-        PairWalk<R> walk(wide, allIn, weighted || g.e1 == g.e2,
-                         weighted ? 0 : uniform(sStart[g.e1]),
-                         weighted ? n : uniform(sCnt[g.e1]),
-                         weighted ? 0 : uniform(sStart[g.e2]),
-                         weighted ? n : uniform(sCnt[g.e2]), S.P, S.M,
-                         S.QUEUE, grc, grc2);
-        if (walk.dp.npairs == 0)
-        {
-            __syncthreads();
-            continue;
-        }
         Members<R, MAXM> M;
         load_members(MP, nmem, M);
         int const nrec = rec && (gi - ed.g0) < kRecordGroups
@@ -501,6 +489,13 @@ __device__ __forceinline__ void force_backward_body(ForceArgs const& a)
             __syncthreads();
             continue;
         }
+        // Weighted type: all unordered pairs of the whole list.
+        PairWalk<R> walk(wide, allIn, weighted || g.e1 == g.e2,
+                         weighted ? 0 : uniform(sStart[g.e1]),
+                         weighted ? n : uniform(sCnt[g.e1]),
+                         weighted ? 0 : uniform(sStart[g.e2]),
+                         weighted ? n : uniform(sCnt[g.e2]), S.P, S.M,
+                         S.QUEUE, grc, grc2);
         walk.run([&](int e, int count) {
             if (lane < count)
                 triplet_backward<CT, GENPOW, MAXM>(gi, S, e & 0xffff, e >> 16,
