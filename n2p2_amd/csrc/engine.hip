@@ -970,6 +970,15 @@ int pairRecordCap(int cap)
     return kRecordGroups + (int)std::min<int64_t>(4096, (all + 63) / 64 * 64);
 }
 
+// Atoms up to which symmetry functions without a pair record (FP64) run a block
+// per group instead of one per atom: one wave per atom leaves most wave slots
+// empty and its groups run one after another, a block per group stages the
+// neighbours again.  One per atom against one per group: 192 water atoms 43
+// and 22 us, 1,536 58 and 45, 2,304 84 and 71, 3,000 77 and 78, 5,900 146 and
+// 156; B/C/N 192 atoms 52 and 17, 1,536 72 and 56, 2,304 83 and 73, 4,500 124
+// and 146.
+constexpr int kSplitAtoms = 2048;
+
 // Whether SF evaluations of this context record the passing pairs for the
 // force kernel: the mixed path, specialised or generic, of every model
 // whose element chunks fit the record's group counts.
@@ -1016,6 +1025,9 @@ void computeSF(hdnnp_ctx* c, bool raw)
         a.pcap = pc;
     }
     c->pairsValid = rec;
+    a.parts = 1;
+    if (!rec && c->n <= kSplitAtoms)
+        for (auto const& e : c->flat.elem) a.parts = std::max(a.parts, e.ng);
     hipEvent_t ev = nullptr;
     c->begin(K_SYMFUNC, ev);
     // Raw (unscaled) evaluations use the same kernels as scaled ones, so
@@ -1025,7 +1037,8 @@ void computeSF(hdnnp_ctx* c, bool raw)
     if (pk.sf && c->n > 0)
     {
         void* params[] = {&a};
-        hipCheck(hipModuleLaunchKernel(pk.sf, (unsigned)c->n, 1, 1, 64, 1, 1,
+        hipCheck(hipModuleLaunchKernel(pk.sf, (unsigned)c->n,
+                                       (unsigned)a.parts, 1, 64, 1, 1,
                                        (unsigned)sf_forward_lds_bytes(c->T,
                                                                       cap,
                                                                       fp32),

@@ -29,6 +29,9 @@ struct SFArgs
     // staged indices j | k << 8.
     unsigned short* pairs;
     int pcap;
+    // Blocks per atom: 1, or at least every element's number of groups, one
+    // group each (no pair record then).
+    int parts;
 };
 
 struct ForceArgs

@@ -184,10 +184,11 @@ template <int MAXM, int CT, typename R>
 void launch_fwd(SFArgs const& a, hipStream_t s)
 {
     size_t const shm = sf_forward_lds_bytes(a.T, a.cap, a.fp32);
+    dim3 const grid(a.n, a.parts);
     if (a.T.genpow)
-        k_sf_forward<MAXM, CT, true, R><<<a.n, 64, shm, s>>>(a);
+        k_sf_forward<MAXM, CT, true, R><<<grid, 64, shm, s>>>(a);
     else
-        k_sf_forward<MAXM, CT, false, R><<<a.n, 64, shm, s>>>(a);
+        k_sf_forward<MAXM, CT, false, R><<<grid, 64, shm, s>>>(a);
 }
 
 template <typename R>

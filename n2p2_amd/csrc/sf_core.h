@@ -256,6 +256,14 @@ __device__ __forceinline__ void sf_forward_body(SFArgs const& a)
     ElemDesc const& ed = T.elem[ec];
     int const s0 = a.off[i];
     int const n = a.cnt[i];
+    // Few atoms: a block per group (SFArgs::parts).
+    int g0 = ed.g0, g1 = ed.g0 + ed.ng;
+    if (a.parts > 1)
+    {
+        g0 += (int)blockIdx.y;
+        if (g0 >= g1) return;
+        g1 = g0 + 1;
+    }
 
     stage_by_element(a, S, s0, n, sStart, sCnt);
 
@@ -272,7 +280,7 @@ __device__ __forceinline__ void sf_forward_body(SFArgs const& a)
     bool wCached = false;
     bool allIn = false;          // every neighbour inside rcCached
     double* __restrict__ Gi = a.G + (size_t)i * a.ldG;
-    for (int gi = ed.g0; gi < ed.g0 + ed.ng; ++gi)
+    for (int gi = g0; gi < g1; ++gi)
     {
         GroupDesc const g = T.group[gi];
         CutCfg const cc = HDNNP_CUT(T.cfg[ed.cfg0 + g.cfg]);
