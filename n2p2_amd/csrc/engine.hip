@@ -551,21 +551,6 @@ void listBuilt(hdnnp_ctx* c, bool partner)
     launchPartner(c);
 }
 
-// The host's copy of a build's statistics: dStats is cleared when it is made
-// and by every read.
-void ensureStats(hdnnp_ctx* c)
-{
-    if (!c->hStats)
-        hipCheck(hipHostMalloc((void**)&c->hStats, 4 * sizeof(int), 0),
-                 "hipHostMalloc");
-    if (c->dStats.cap < 4)
-    {
-        c->dStats.ensure(4);
-        hipCheck(hipMemsetAsync(c->dStats.p, 0, 4 * sizeof(int), c->stream),
-                 "memset");
-    }
-}
-
 // hstat[0] = largest of n counts, hstat[1..3] = the builder's flags (waits).
 void readStats(hdnnp_ctx* c, const int* count, int n, int* hstat)
 {
@@ -691,8 +676,6 @@ void buildBatchNeighborList(hdnnp_ctx* c, double rc, bool partner)
                                  c->dCells.p, s), "batch extent");
     c->dCount.ensure(n);
     c->dOff.ensure(n + 1);
-    c->dStats.ensure(4);
-    ensureStats(c);
     fillSlabs(c, rc, c->dCells.p, BatchCell{});
     c->end(K_NEIGHBOR, ev0);
     c->ownOrder = true;
@@ -729,7 +712,6 @@ bool buildSmallNeighborList(hdnnp_ctx* c, double rc, bool partner)
     c->begin(K_NEIGHBOR, ev0);
     c->dCount.ensure(n);
     c->dOff.ensure(n + 1);
-    ensureStats(c);
     fillSlabs(c, rc, nullptr, one);
     if (c->maxNeigh > 8192)
         throw Error(HDNNP_E_CAPACITY,
@@ -828,7 +810,6 @@ void buildNeighborList(hdnnp_ctx* c, double rc, bool partner = true)
     c->dCellAtoms.ensure(n);
     c->dCount.ensure(n);
     c->dOff.ensure(n + 1);
-    ensureStats(c);
     c->dBlockSums.ensure((std::max(n, ncell) + 1023) / 1024 + 1);
     c->dTotal.ensure(1);
     hipCheck(hipMemsetAsync(c->dCellCount.p, 0, ncell * sizeof(int), s), "memset");
@@ -1549,8 +1530,15 @@ int hdnnp_ctx_create(const hdnnp_model* m, int device, hdnnp_ctx** out)
         c->dSumScratch.ensure(ns);
         hipCheck(hipMemsetAsync(c->dSumScratch.p, 0, ns * sizeof(double),
                                 c->stream), "memset");
-        hipCheck(hipHostMalloc((void**)&c->hEnergy, sizeof(double), 0),
+        // Statistics of list builds (dStats: cleared here and by every read)
+        // and the energy, in one pinned block.
+        c->dStats.ensure(4);
+        hipCheck(hipMemsetAsync(c->dStats.p, 0, 4 * sizeof(int), c->stream),
+                 "memset");
+        hipCheck(hipHostMalloc((void**)&c->hEnergy,
+                               sizeof(double) + 4 * sizeof(int), 0),
                  "hipHostMalloc");
+        c->hStats = (int*)(c->hEnergy + 1);
         *out = c.release();
     });
 }
@@ -1573,7 +1561,6 @@ void hdnnp_ctx_destroy(hdnnp_ctx* c)
     c->dMember.release(); c->dRun.release(); c->dScale.release(); c->dPairGroups.release();
     c->dCompGroup.release(); c->dCompMember.release();
     c->dCompRun.release(); c->dCompAng.release();
-    if (c->hStats) (void)hipHostFree(c->hStats);
     if (c->hEnergy) (void)hipHostFree(c->hEnergy);
     c->dSumScratch.release();
     c->dPairCount.release(); c->dWeights.release();
@@ -3145,8 +3132,7 @@ int hdnnp_set_neighbor_list(hdnnp_ctx* c, int64_t ncentre,
         c->dScatSrc.ensure((size_t)n + (size_t)M);
         c->dCslot.ensure(3 * m1);    // the forces' later place holds dr
         c->dRank.ensure(n);
-        ensureStats(c);
-        up(c->dScatSrc.p, nbr_index, (size_t)M);
+            up(c->dScatSrc.p, nbr_index, (size_t)M);
         up(c->dElemAtom.p + n, nbr_elem, (size_t)M);
         up(c->dCslot.p, dr, 3 * (size_t)M);
         hipCheck(launch_ext_entries(n, (int)M, ne, c->dScatSrc.p,
