@@ -737,7 +737,6 @@ void buildNeighborList(hdnnp_ctx* c, double rc, bool partner = true)
         return;
     }
     if (buildSmallNeighborList(c, rc, partner)) return;
-    c->ownOrder = false;
     NLParams& p = c->nl;
     p = NLParams{};
     p.n = (int)c->n;
@@ -803,6 +802,9 @@ void buildNeighborList(hdnnp_ctx* c, double rc, bool partner = true)
     hipStream_t s = c->stream;
     hipEvent_t ev0 = nullptr;
     c->begin(K_NEIGHBOR, ev0);
+    // Not before the checks above: a list they refuse leaves the one before
+    // as it is, with its own order.
+    c->ownOrder = false;
     c->dCellOfAtom.ensure(n);
     c->dRank.ensure(n);
     c->dCellCount.ensure(ncell);
