@@ -188,6 +188,13 @@ struct hdnnp_ctx
     DBuf<double> dG, dE, dEdG, dScratch, dCslot, dCself, dF, dEnergy, dStatOut;
     DBuf<int> dEw;
     bool haveSF = false, haveNN = false, haveNNDeriv = false;
+    // No list, and nothing evaluated on one: from before the first change a
+    // build makes until it has succeeded.
+    void dropList()
+    {
+        haveNL = haveSF = haveNN = haveNNDeriv = false;
+        partnerMissing = false;
+    }
     double energy = 0.0;
     int precision = HDNNP_PRECISION_FP64;
     // Pair record of the mixed path: the SF kernel writes the passing
@@ -448,6 +455,14 @@ void requireNL(hdnnp_ctx* c)
         throw Error(HDNNP_E_INVALID, "ERROR: Neighbor list not calculated.\n");
 }
 
+// An MD run whose last list rebuild failed has positions but no list.
+void requireMdList(hdnnp_ctx* c)
+{
+    if (!c->haveNL)
+        throw Error(HDNNP_E_INVALID, "ERROR: The MD run has no neighbour list "
+                                     "(its last rebuild failed).\n");
+}
+
 // Structure::calculateInverseBox (Structure.cpp:519-545).
 void inverseBox(double const b[3][3], double ib[3][3])
 {
@@ -669,6 +684,7 @@ void buildBatchNeighborList(hdnnp_ctx* c, double rc, bool partner)
     }
     hipEvent_t ev0 = nullptr;
     c->begin(K_NEIGHBOR, ev0);
+    c->dropList();
     c->dCells.ensure(ns);
     hipCheck(hipMemcpyAsync(c->dCells.p, cells.data(), ns * sizeof(BatchCell),
                             hipMemcpyHostToDevice, s), "cells");
@@ -683,7 +699,6 @@ void buildBatchNeighborList(hdnnp_ctx* c, double rc, bool partner)
     c->slabLayout = true;
     c->Mvalid = false;
     c->haveNL = true;
-    c->haveSF = c->haveNN = c->haveNNDeriv = false;
 }
 
 // A single structure of at most kSmallList atoms without cells; false if it
@@ -710,6 +725,7 @@ bool buildSmallNeighborList(hdnnp_ctx* c, double rc, bool partner)
     }
     hipEvent_t ev0 = nullptr;
     c->begin(K_NEIGHBOR, ev0);
+    c->dropList();
     c->dCount.ensure(n);
     c->dOff.ensure(n + 1);
     fillSlabs(c, rc, nullptr, one);
@@ -722,7 +738,6 @@ bool buildSmallNeighborList(hdnnp_ctx* c, double rc, bool partner)
     c->slabLayout = true;
     c->Mvalid = false;
     c->haveNL = true;
-    c->haveSF = c->haveNN = c->haveNNDeriv = false;
     return true;
 }
 
@@ -804,6 +819,7 @@ void buildNeighborList(hdnnp_ctx* c, double rc, bool partner = true)
     c->begin(K_NEIGHBOR, ev0);
     // Not before the checks above: a list they refuse leaves the one before
     // as it is, with its own order.
+    c->dropList();
     c->ownOrder = false;
     c->dCellOfAtom.ensure(n);
     c->dRank.ensure(n);
@@ -921,7 +937,6 @@ void buildNeighborList(hdnnp_ctx* c, double rc, bool partner = true)
     // slab bounds it; a rebuild above raised the slab if it was exceeded).
     c->maxNeigh = cellKernels ? std::min(maxc, c->slab) : maxc;
     c->haveNL = true;
-    c->haveSF = c->haveNN = c->haveNNDeriv = false;
 }
 
 // Total neighbour-list entries (summed from the per-atom counts once per
@@ -1935,7 +1950,7 @@ int hdnnp_ctx_set_tuning(hdnnp_ctx* c, const int* in4)
 static void dropStructure(hdnnp_ctx* c)
 {
     c->waitPartner();
-    c->partnerMissing = false;
+    c->dropList();
     c->sync();   // the side stream no longer reads the list buffers
     mdEnd(c);
     c->n = 0;
@@ -1945,7 +1960,6 @@ static void dropStructure(hdnnp_ctx* c)
     c->batched = false;
     c->nstruct = 0;
     c->hostPosValid = false;
-    c->haveNL = c->haveSF = c->haveNN = c->haveNNDeriv = false;
 }
 
 // Atoms, elements and per-element atom lists of a structure or a batch.
@@ -2102,7 +2116,7 @@ int hdnnp_set_positions(hdnnp_ctx* c, const double* r)
                                 hipMemcpyHostToDevice, c->stream), "positions");
         c->hR.assign(r, r + 3 * c->n);
         c->hostPosValid = true;
-        c->haveNL = c->haveSF = c->haveNN = c->haveNNDeriv = false;
+        c->dropList();
     });
 }
 
@@ -2119,7 +2133,7 @@ int hdnnp_set_positions_device(hdnnp_ctx* c, const double* r_device)
                                 hipMemcpyDeviceToDevice, c->stream),
                  "positions");
         c->hostPosValid = false;
-        c->haveNL = c->haveSF = c->haveNN = c->haveNNDeriv = false;
+        c->dropList();
     });
 }
 
@@ -2401,6 +2415,7 @@ int hdnnp_md_run(hdnnp_ctx* c, int64_t nsteps, double* epot, double* ekin)
                                          "call ends the run).\n");
         if (nsteps < 0 || nsteps > 100000000)
             throw Error(HDNNP_E_INVALID, "ERROR: Bad step count.\n");
+        requireMdList(c);
         c->setDevice();
         auto& m = c->md;
         int const need = (int)std::max<int64_t>(nsteps, 1);
@@ -2647,6 +2662,8 @@ int hdnnp_mts_run(hdnnp_ctx* sur, int64_t nouter, double* epot, double* ekin,
                                          "(hdnnp_mts_init).\n");
         if (nouter < 0 || nouter > 100000000)
             throw Error(HDNNP_E_INVALID, "ERROR: Bad step count.\n");
+        requireMdList(sur);
+        requireMdList(S.full);
         sur->setDevice();
         int const need = (int)std::max<int64_t>(nouter, 1);
         if (need > S.recCap)
@@ -3178,7 +3195,6 @@ int hdnnp_set_neighbor_list(hdnnp_ctx* c, int64_t ncentre,
         c->hostPosValid = false;
         c->n = n;
         c->haveNL = true;
-        c->haveSF = c->haveNN = c->haveNNDeriv = false;
     });
 }
 

@@ -63,6 +63,11 @@ def test_neighbor_limit(model, rc):
     if rc > 25.0:
         with pytest.raises(RuntimeError, match="8192"):
             ctx.calculate_neighbor_list(rc)
+        # The refused list's counts are on the device: nothing may run on them.
+        for call in (ctx.calculate_symmetry_function_groups, ctx.neighbors):
+            with pytest.raises(RuntimeError, match="not calculated"):
+                call()
+        _check(ctx, om, r, elem, box, 12.0)
         ctx.set_structure(r, elem, box)
         _check(ctx, om, r, elem, box, 12.0)
         return
