@@ -1234,6 +1234,7 @@ void mdEnd(hdnnp_ctx* c)
     if (!c->md.on) return;
     mdDropGraphs(c);
     c->md.on = false;
+    c->dropList();   // the filtered list has no partner map of its own
 }
 
 void mdDropGraphs(hdnnp_ctx* c)

@@ -74,3 +74,16 @@ def test_failed_md_start(model):
         ctx.md_run(1)
     ctx.md_init([10.8, 12.0, 14.0], 0.1, skin=1.0)
     ctx.md_run(2)
+
+
+def test_end_of_md_drops_the_filtered_list(model):
+    r, elem, box = W.random_structure(300, seed=5)
+    ctx = engine.Context(model)
+    ctx.set_structure(r, elem, box)
+    e = ctx.evaluate(engine.FORCES_CONSISTENT)
+    ctx.md_init([10.8, 12.0, 14.0], 0.1, skin=1.0)
+    with pytest.raises(RuntimeError, match="60 periodic images"):
+        ctx.calculate_neighbor_list(70.0 * box[0, 0])    # ends the run
+    with pytest.raises(RuntimeError):
+        ctx.calculate_forces(engine.FORCES_CONSISTENT)
+    assert abs(ctx.evaluate(engine.FORCES_CONSISTENT) - e) < 1e-9 * abs(e)
