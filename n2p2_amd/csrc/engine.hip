@@ -195,6 +195,9 @@ struct hdnnp_ctx
         haveNL = haveSF = haveNN = haveNNDeriv = false;
         partnerMissing = false;
     }
+    // Entries of the list whose forces dF, dCself and dCslot hold; -1: none
+    // for this structure.
+    int64_t forcesOf = -1;
     double energy = 0.0;
     int precision = HDNNP_PRECISION_FP64;
     // Pair record of the mixed path: the SF kernel writes the passing
@@ -1149,6 +1152,7 @@ void computeForces(hdnnp_ctx* c, int mode, bool wait = true)
         throw Error(HDNNP_E_CAPACITY,
                     "ERROR: Too many neighbours per atom for the force "
                     "kernel's LDS staging.\n");
+    c->forcesOf = -1;
     c->dCslot.ensure(3 * (size_t)std::max<int64_t>(c->entryCap, 1));
     c->dCself.ensure(3 * (size_t)c->n);
     c->dF.ensure(3 * (size_t)c->n);
@@ -1189,6 +1193,7 @@ void computeForces(hdnnp_ctx* c, int mode, bool wait = true)
     c->end(K_FORCE, ev);
     if (partner) launchPartner(c);
     launchGather(c, mode);
+    c->forcesOf = c->entryCap;
     if (wait) c->sync();
 }
 
@@ -1961,6 +1966,7 @@ static void dropStructure(hdnnp_ctx* c)
     c->batched = false;
     c->nstruct = 0;
     c->hostPosValid = false;
+    c->forcesOf = -1;
 }
 
 // Atoms, elements and per-element atom lists of a structure or a batch.
@@ -2318,7 +2324,8 @@ int hdnnp_get_forces(hdnnp_ctx* c, double* f)
             throw Error(HDNNP_E_INVALID, "ERROR: Forces of a caller-given "
                                          "neighbour list are scattered with "
                                          "hdnnp_get_scattered_forces.\n");
-        if (!c->dF.p) throw Error(HDNNP_E_INVALID, "ERROR: No forces.\n");
+        if (c->forcesOf < 0)
+            throw Error(HDNNP_E_INVALID, "ERROR: No forces.\n");
         c->setDevice();
         copyOut(c, f, c->dF.p, 3 * (size_t)c->n);
         c->sync();
@@ -3152,7 +3159,7 @@ int hdnnp_set_neighbor_list(hdnnp_ctx* c, int64_t ncentre,
         c->dScatSrc.ensure((size_t)n + (size_t)M);
         c->dCslot.ensure(3 * m1);    // the forces' later place holds dr
         c->dRank.ensure(n);
-            up(c->dScatSrc.p, nbr_index, (size_t)M);
+        up(c->dScatSrc.p, nbr_index, (size_t)M);
         up(c->dElemAtom.p + n, nbr_elem, (size_t)M);
         up(c->dCslot.p, dr, 3 * (size_t)M);
         hipCheck(launch_ext_entries(n, (int)M, ne, c->dScatSrc.p,
@@ -3205,7 +3212,7 @@ int hdnnp_get_scattered_forces(hdnnp_ctx* c, int64_t nout, double* f)
         if (!c || !c->externalNL)
             throw Error(HDNNP_E_INVALID, "ERROR: No caller-given neighbour "
                                          "list.\n");
-        if (!c->dCself.p || !c->dCslot.p)
+        if (c->forcesOf < 0)
             throw Error(HDNNP_E_INVALID, "ERROR: No forces.\n");
         if (nout < c->extTargets)
             throw Error(HDNNP_E_INVALID, "ERROR: Centre or neighbour index "
@@ -3263,7 +3270,7 @@ int hdnnp_get_scattered_forces_noalloc(hdnnp_ctx* c, int64_t nout, double* f)
         if (!c || !c->externalNL)
             throw Error(HDNNP_E_INVALID, "ERROR: No caller-given neighbour "
                                          "list.\n");
-        if (!c->dCself.p || !c->dCslot.p)
+        if (c->forcesOf < 0)
             throw Error(HDNNP_E_INVALID, "ERROR: No forces.\n");
         if (nout < c->extTargets)
             throw Error(HDNNP_E_INVALID, "ERROR: Centre or neighbour index "
@@ -3295,7 +3302,7 @@ int hdnnp_get_pair_forces(hdnnp_ctx* c, double* self_forces,
                           double* pair_forces)
 {
     return guarded([&]() {
-        if (!c->dF.p || !c->haveNL)
+        if (!c->haveNL || c->forcesOf != c->entryCap)
             throw Error(HDNNP_E_INVALID, "ERROR: No forces.\n");
         c->setDevice();
         copyOut(c, self_forces, c->dCself.p, 3 * (size_t)c->n);

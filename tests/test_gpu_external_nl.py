@@ -157,3 +157,42 @@ def test_interface_lammps_driver(workdir, tmp_path, case):
     say("  energy rel %.3g, folded force max %.3g" % (de, df))
     assert de <= 1e-10
     assert df <= 1e-9
+
+
+def test_forces_of_another_list_are_refused(workdir):
+    """A second, larger list on the same context: its entries lie where slot
+    forces will be, and the centres' forces are still those of the first list,
+    so nothing is given out before the forces are computed."""
+    d, r, e, box = cases.water_case(workdir)
+    m = engine.Model.load_dir(d)
+    x, el, owner, nl = ghost_domain(r, e, box, m.max_cutoff)
+    off, idx, dr = full_lists(x, nl, m.max_cutoff)
+    ctx = engine.Context(m)
+    k = 64
+    ctx.set_neighbor_list(el[:k], off[:k + 1], idx[:off[k]],
+                          el[idx[:off[k]]], dr[:off[k]])
+    ctx.evaluate(engine.FORCES_CONSISTENT)
+    ctx.scattered_forces(len(x))
+    ctx.set_neighbor_list(el[:nl], off, idx, el[idx], dr)
+
+    def refused():
+        for call in (lambda: ctx.scattered_forces(len(x)),
+                     lambda: ctx.scattered_forces_noalloc(len(x)),
+                     ctx.pair_forces):
+            with pytest.raises(RuntimeError, match="No forces"):
+                call()
+
+    refused()
+    ctx.evaluate(-1)
+    refused()
+    ctx.evaluate(engine.FORCES_CONSISTENT)
+    f = ctx.scattered_forces(len(x))
+    assert np.array_equal(f, ctx.scattered_forces_noalloc(len(x)))
+    # A structure instead of the list.
+    ctx.set_structure(np.concatenate([r, r + 0.7]), np.concatenate([e, e]),
+                      2.0 * box)
+    with pytest.raises(RuntimeError, match="No forces"):
+        ctx.forces()
+    with pytest.raises(RuntimeError, match="No forces"):
+        ctx.pair_forces()
+    ctx.close()
