@@ -86,18 +86,20 @@ __device__ __forceinline__ void sincospi01(float x, float& s, float& c)
     c = __builtin_amdgcn_cosf(rev);
 }
 
-// sin and cos of pi r iw (FP32: half the scale as the revolutions, which
-// rounds as r iw / 2 does).
+// sin and cos of pi r iw, r iw in [0, 1] (FP32: half the scale as the
+// revolutions, which rounds as r iw / 2 does).  Two neighbours at one place
+// have r = 0 1/sqrt(0), NaN, for 0; FP32: the clamp, a modifier of the
+// multiplication, makes it that.
 __device__ __forceinline__ void sincospi_scaled(double r, double iw, double& s,
                                                 double& c)
 {
-    sincospi01(r * iw, s, c);
+    sincospi01(fmax(r, 0.0) * iw, s, c);
 }
 
 __device__ __forceinline__ void sincospi_scaled(float r, float iw, float& s,
                                                 float& c)
 {
-    float const rev = r * (0.5f * iw);
+    float const rev = fminf(fmaxf(r * (0.5f * iw), 0.0f), 1.0f);
     s = __builtin_amdgcn_sinf(rev);
     c = __builtin_amdgcn_cosf(rev);
 }
