@@ -177,7 +177,10 @@ void emit_forward_case(std::ostringstream& o, int gi, GroupDesc const& g,
                        Model::Flat const& F)
 {
     bool const wide = (g.type == 9);
-    o << "    case " << gi << ":\n    {\n        R vp = R(0);\n";
+    // An atom on its neighbour has no angle (NaN): the power chain's fmax
+    // would drop that, so the factor of all members carries it.
+    o << "    case " << gi << ":\n    {\n        R vp = R(0);\n"
+      << "        R const pn_ = fma(R(0), costijk, pfc);\n";
     for (int ri = 0; ri < g.nrun; ++ri)
     {
         LamRun const& r = F.run[g.run0 + ri];
@@ -186,7 +189,7 @@ void emit_forward_case(std::ostringstream& o, int gi, GroupDesc const& g,
             o << "        {\n";
             emit_exp_sum(o, r, wide);
             o << "        vp = exp_scaled(exp_factor(" << lit(r.eta)
-              << ") * s_) * pfc;\n        }\n";
+              << ") * s_) * pn_;\n        }\n";
         }
         o << "        {\n        R const pl = " << plambda(r.lambda) << ";\n"
           << "        R P, X = fmax(pl, R(0));\n"

@@ -1,6 +1,8 @@
-"""Two atoms at one place.  Every other atom sees two neighbours at distance 0
-from each other, which is no special case: G and energies are the oracle's
-(bounds of test_gpu_pair_search.py)."""
+"""Two atoms at one place.  Their own symmetry functions have no value (the
+angle at r = 0), so the specialised kernels must give NaN there and for the
+energy, as the formula and the oracle do; every other atom sees two neighbours
+at distance 0 from each other, which is no special case: G and energies are the
+oracle's (bounds of test_gpu_pair_search.py)."""
 import os
 
 import numpy as np
@@ -35,10 +37,14 @@ def test_coincident_atoms(tmp_path, types, cut):
             ctx.set_specialized(spec)
             ctx.set_structure(r, elem, box)
             e = ctx.evaluate(engine.FORCES_CONSISTENT)
-            g, ea = ctx.G(), ctx.atomic_energies()
+            g, ea, f = ctx.G(), ctx.atomic_energies(), ctx.forces()
             bad = np.isnan(g).any(1)
             print("[gpu-coincident]", types, cut, prec, spec, e,
                   np.flatnonzero(bad), flush=True)
+            if spec:
+                assert np.isnan(e)
+                assert np.array_equal(bad, two)
+                assert np.isnan(f[two]).all()
             assert not bad[~two].any()
             err = np.abs(g[~two][:, :og.shape[1]] - og).max()
             assert err <= TOL[prec][0] * np.abs(og).max()
