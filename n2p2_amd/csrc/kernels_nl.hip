@@ -270,8 +270,8 @@ __global__ __launch_bounds__(64) void k_nl(
 
 // Cell kernels: one workgroup of four waves per cell.  The atoms of the
 // cell's (2m+1)^3 neighbour cells (m = 1 when cells are at least rc wide)
-// are staged once in LDS as keys and FP32 positions relative to the cell's
-// first atom; each wave then takes one atom of the cell at a time and tests
+// are staged once in LDS as keys and FP32 positions relative to one atom of
+// the cell; each wave then takes one atom of the cell at a time and tests
 // all staged candidates, 64 per step.  MODE 0 counts hits.  MODE 1 first sorts
 // the candidates by (j, image), the reference's loop order, so that an atom's
 // hits come in list order and are written directly.
@@ -422,10 +422,19 @@ __global__ __launch_bounds__(256) void k_nl_cell(
         __syncthreads();
     }
     int const a0 = cellStart[cell];
+    // The first atom with finite coordinates (one without would hide the
+    // others' neighbours); a cell of none has no neighbours at all.
     double org[3];
+    for (int a = 0; a < nAt; ++a)
     {
-        int const i0 = cellAtoms[a0];
-        for (int k = 0; k < 3; ++k) org[k] = r[3 * (size_t)i0 + k];
+        int const i0 = cellAtoms[a0 + a];
+        bool finite = true;
+        for (int k = 0; k < 3; ++k)
+        {
+            org[k] = r[3 * (size_t)i0 + k];
+            finite &= __builtin_isfinite(org[k]);
+        }
+        if (finite) break;
     }
     float far = 0.0f;
     for (int t = tid; t < total; t += 256)
