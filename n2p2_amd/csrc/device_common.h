@@ -719,10 +719,11 @@ constexpr int kPairQueueAlloc = kPairQueue + 4;
 typedef float Float4V __attribute__((ext_vector_type(4)));
 
 // Staged position and half its negative square, (x, y, z, -r^2 / 2), as the
-// pair search reads it; -1e30 in place of the square keeps the neighbour out
-// (r >= rc).  FP32 records give it as it is read, FP64 ones keep a float copy
-// M.
-constexpr float kOutside = -1e30f;
+// pair search reads it; minus infinity in place of the square keeps the
+// neighbour out (r >= rc) wherever it is: the sum is that or NaN, also where
+// products of coordinates overflow.  FP32 records give it as it is read, FP64
+// ones keep a float copy M.
+constexpr float kOutside = -__builtin_inff();
 
 __device__ __forceinline__ Float4V search_row(Vec4<float> const* P,
                                               Float4V const*, float rc, int t)
@@ -756,9 +757,10 @@ __device__ __forceinline__ Float4V search_entry(double4 const& g)
 // The distances are FP32 with an error below 2e-6 rc^2 (15 roundings of terms
 // up to 1.5 rc^2, h and, on the FP64 path, the rounded positions included),
 // so pairs up to 8e-6 rc^2 beyond are let through and the evaluation takes
-// f_c(rjk) = 0 for those (rij, rik < rc hold exactly: h).  One neighbour pair per lane and step (differences,
-// squares, index arithmetic and queue: 37 vector instructions per 64 pairs
-// instead of about 12) made the search 40% of the symmetry-function kernel.
+// f_c(rjk) = 0 for those (rij, rik < rc hold exactly: h).  One neighbour pair
+// per lane and step (differences, squares, index arithmetic and queue: 37
+// vector instructions per 64 pairs instead of about 12) made the search 40% of
+// the symmetry-function kernel.
 //
 // Wide: no distance to search; if every neighbour of the list is inside rc
 // (direct) the pairs go to the lanes as they come, else through the queue.

@@ -196,3 +196,38 @@ def test_forces_of_another_list_are_refused(workdir):
     with pytest.raises(RuntimeError, match="No forces"):
         ctx.pair_forces()
     ctx.close()
+
+
+@pytest.mark.parametrize("far", [1e10, 1e16, 1e25, 1e200])
+@pytest.mark.parametrize("prec", [engine.PRECISION_FP64,
+                                  engine.PRECISION_MIXED])
+def test_entries_far_outside_the_cutoff(workdir, prec, far):
+    """A list padded with entries at one far place, as a caller with rows of a
+    fixed length gives it: symmetry functions and forces are those of the list
+    without them to the order of the sums (1e-12 of the largest in FP64; 2e-6 in
+    FP32, 16 eps), and the padding receives none."""
+    tol = 1e-12 if prec == engine.PRECISION_FP64 else 2e-6
+    d, r, e, box = cases.water_case(workdir)
+    m = engine.Model.load_dir(d)
+    x, el, owner, nl = ghost_domain(r, e, box, m.max_cutoff)
+    off, idx, dr = full_lists(x, nl, m.max_cutoff)
+    keep = np.insert(np.ones(len(idx), bool), np.repeat(off[1:], 2), False)
+    pad = np.insert(idx, np.repeat(off[1:], 2), len(x))
+    pdr = np.insert(dr, np.repeat(off[1:], 2), far, axis=0)
+    pel = np.append(el, el[0])
+    out = []
+    for o, i, v in ((off, idx, dr),
+                    (off + 2 * np.arange(len(off)), pad, pdr)):
+        ctx = engine.Context(m)
+        ctx.set_precision(prec)
+        ctx.set_neighbor_list(el[:nl], o, i, pel[i], v)
+        ctx.evaluate(engine.FORCES_CONSISTENT)
+        out.append((ctx.G(), ctx.scattered_forces(len(x) + 1),
+                    ctx.pair_forces()[1]))
+        ctx.close()
+    say("far %g, precision %d: %d entries of padding"
+        % (far, prec, (~keep).sum()))
+    (g, f, p), (gp, fp, pp) = out
+    for a, b in ((g, gp), (f, fp), (p, pp[keep])):
+        assert np.abs(a - b).max() <= tol * np.abs(a).max()
+    assert not pp[~keep].any()
