@@ -2787,15 +2787,14 @@ int hdnnp_train_gradient(hdnnp_ctx* c, const double* f_ref, double e_ref,
         A.wE = w_e;
         A.cF = -2.0 * w_f / (3.0 * (double)n);
         A.cap = std::max(c->maxNeigh, 1);
+        if (train_u_lds_bytes(A.cap) > kLdsPerWorkgroup
+            || (c->T.ncgroup > 0
+                && train_u_compact_lds_bytes(c->T, A.cap) > 65536))
+            throw Error(HDNNP_E_CAPACITY,
+                        "ERROR: Too many neighbours per atom for the "
+                        "training kernels' LDS staging.\n");
         hipCheck(launch_train_u(A, s), "train u");
-        {
-            int const cap = std::max(c->maxNeigh, 1);
-            if (c->T.ncgroup > 0 && train_u_compact_lds_bytes(c->T, cap) > 65536)
-                throw Error(HDNNP_E_CAPACITY,
-                            "ERROR: Too many neighbours per atom for the "
-                            "compact training kernel's LDS staging.\n");
-            hipCheck(launch_train_u_compact(A, cap, s), "train u (compact)");
-        }
+        hipCheck(launch_train_u_compact(A, A.cap, s), "train u (compact)");
         {
             int const* atoms[kMaxElements] = {};
             int na[kMaxElements] = {};

@@ -117,6 +117,9 @@ int train_atoms_per_block();
 int train_atoms_per_grad_block(ElemDesc const& ed);
 size_t train_lds_per_atom(ElemDesc const& ed);
 hipError_t launch_train_u(TrainArgs const& A, hipStream_t s);
+// LDS of launch_train_u at `cap` neighbours, and what a workgroup may have.
+size_t train_u_lds_bytes(int cap);
+constexpr size_t kLdsPerWorkgroup = 160 * 1024;
 // The compact SF types' part of u (after launch_train_u); cap = the largest
 // neighbour count.
 hipError_t launch_train_u_compact(TrainArgs const& A, int cap, hipStream_t s);

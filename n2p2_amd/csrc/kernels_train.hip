@@ -364,10 +364,16 @@ __global__ __launch_bounds__(64) void k_train_u(TrainArgs A)
     }
 }
 
+// The static LDS of k_train_u, rounded up.
+constexpr size_t kTrainStatic = 2048;
+static_assert(kMaxMembers * sizeof(MParam<double>)
+                  + 2 * kMaxElements * sizeof(int) <= kTrainStatic,
+              "static LDS of k_train_u");
+
 template <int MAXM>
 void launch_train_u_m(TrainArgs const& A, hipStream_t s)
 {
-    size_t const shm = force_list_lds_bytes(A.cap, 0);
+    size_t const shm = train_u_lds_bytes(A.cap) - kTrainStatic;
     if (A.T.genpow)
         HDNNP_CUTOFF_DISPATCH(A.T.cutType,
             (k_train_u<MAXM, kCT, true><<<A.n, 64, shm, s>>>(A)));
@@ -885,11 +891,17 @@ size_t train_lds_per_atom(ElemDesc const& ed)
     return p + 2 * ed.maxwidth;
 }
 
+// 11 doubles per staged neighbour and the pair queue, as the FP64 force kernel
+// before the pair search.  Also on the mixed path, whose force kernel admits
+// lists by 56 bytes per neighbour, up to 1,161: 102 KB here.
+size_t train_u_lds_bytes(int cap)
+{
+    return force_list_lds_bytes(cap, 0) + kTrainStatic;
+}
+
 hipError_t launch_train_u(TrainArgs const& A, hipStream_t s)
 {
     if (A.n <= 0) return hipSuccess;
-    // The LDS of the FP64 force kernel, which ran before on the same list:
-    // 11 doubles per staged neighbour and the pair queue.
     if (A.T.maxGroupMembers <= 8) launch_train_u_m<8>(A, s);
     else launch_train_u_m<kMaxMembers>(A, s);
     return hipGetLastError();
