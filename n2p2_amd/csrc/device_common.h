@@ -718,29 +718,23 @@ constexpr int kPairQueueAlloc = kPairQueue + 4;
 
 typedef float Float4V __attribute__((ext_vector_type(4)));
 
-// Staged position and half its negative square, (x, y, z, -r^2 / 2), as the
-// pair search reads it; minus infinity in place of the square keeps the
-// neighbour out (r >= rc) wherever it is: the sum is that or NaN, also where
-// products of coordinates overflow.  FP32 records give it as it is read, FP64
-// ones keep a float copy M.
+// Position of staged neighbour t in FP32 and half its negative square,
+// (x, y, z, -r^2 / 2), as the pair search reads it; minus infinity in place of
+// the square keeps the neighbour out (r >= rc) wherever it is: the sum is that
+// or NaN, also where products of coordinates overflow.  FP64 records are
+// rounded as they are read: a float copy beside them cost 16 of 64 bytes of LDS
+// per neighbour and with it workgroups per CU (196,608 water atoms 9,790 ->
+// 9,510 us; 8,000 atoms of 366 neighbours, symmetry functions 2,530 -> 2,340
+// and force 4,500 -> 3,710 us).
 constexpr float kOutside = -__builtin_inff();
 
-__device__ __forceinline__ Float4V search_row(Vec4<float> const* P,
-                                              Float4V const*, float rc, int t)
+template <typename R>
+__device__ __forceinline__ Float4V search_row(Vec4<R> const* P, R rc, int t)
 {
-    Vec4<float> const p = P[t];
-    return Float4V{p.x, p.y, p.z, p.w < rc ? -0.5f * (p.w * p.w) : kOutside};
-}
-
-__device__ __forceinline__ Float4V search_row(Vec4<double> const*,
-                                              Float4V const* M, double, int t)
-{
-    return M[t];
-}
-
-__device__ __forceinline__ Float4V search_entry(double4 const& g)
-{
-    return Float4V{(float)g.x, (float)g.y, (float)g.z, kOutside};
+    Vec4<R> const p = P[t];
+    float const r = (float)p.w;
+    return Float4V{(float)p.x, (float)p.y, (float)p.z,
+                   p.w < rc ? -0.5f * (r * r) : kOutside};
 }
 
 // The pairs {j, k} of a group's neighbour blocks that can pass rij, rik < rc
@@ -769,7 +763,6 @@ struct PairWalk
 {
     DiagPairs dp;         // neighbours (wide) or blocks of four (narrow)
     Vec4<R> const* P;
-    Float4V const* M;
     int* Q;
     R rc;
     float thr;
@@ -779,9 +772,9 @@ struct PairWalk
 
     __device__ __forceinline__ PairWalk(bool wide_, bool allIn, bool same,
                                         int a0, int na, int b0, int nb,
-                                        Vec4<R> const* P_, Float4V const* M_,
-                                        int* Q_, R rc_, R rc2)
-        : dp(same, a0, na, b0, nb), P(P_), M(M_), Q(Q_), rc(rc_),
+                                        Vec4<R> const* P_, int* Q_, R rc_,
+                                        R rc2)
+        : dp(same, a0, na, b0, nb), P(P_), Q(Q_), rc(rc_),
           thr(-0.5f * (1.0f + 8e-6f) * (float)rc2), base(0), qn(0), c(0),
           r(0), wide(wide_), direct(wide_ && allIn)
     {
@@ -814,8 +807,8 @@ struct PairWalk
         if (v >= dp.nl) v -= dp.nl;
         int const ja = s0 + 4 * r, kb = l0 + 4 * v + j;
         // Beyond the end (also of the pairs): a neighbour in bounds, kept out.
-        Float4V A = search_row(P, M, rc, min(ja + j, e0));
-        Float4V B = search_row(P, M, rc, min(kb, e1));
+        Float4V A = search_row(P, rc, min(ja + j, e0));
+        Float4V B = search_row(P, rc, min(kb, e1));
         if (ja + j > e0) A.w = kOutside;
         if (kb > e1 || !valid) B.w = kOutside;
         Float4V d = {0.0f, 0.0f, 0.0f, 0.0f};

@@ -82,7 +82,6 @@ struct BLds
                      // (FP64 on both paths): lanes on neighbouring slots
                      // hit neighbouring banks
     int cap;
-    Float4V* M;      // FP64: float copy for the pair search
     int* QUEUE;      // kPairQueue pairs, j | k << 16
 };
 
@@ -156,7 +155,6 @@ __device__ __forceinline__ void stage(ForceArgs const& a, BLds<R> const& S,
                     S.ACC[pos] = 0.0;
                     S.ACC[S.cap + pos] = 0.0;
                     S.ACC[2 * S.cap + pos] = 0.0;
-                    if (sizeof(R) == 8 && S.M) S.M[pos] = search_entry(g);
                 }
                 start[q] += __popcll(mask);
             }
@@ -359,11 +357,7 @@ __device__ __forceinline__ void force_backward_body(ForceArgs const& a)
     S.Q = S.P + cap;
     S.ACC = (double*)(S.Q + cap);
     S.cap = cap;
-    constexpr bool kFloat = sizeof(R) == 4;
-    double* const end = S.ACC + 3 * cap + (cap & 1);    // 16-byte aligned
-    bool const copy = !kFloat && HDNNP_WIDE != 1 && T.narrow;
-    S.M = copy ? (Float4V*)end : nullptr;
-    S.QUEUE = copy ? (int*)(S.M + cap) : (int*)end;
+    S.QUEUE = (int*)(S.ACC + 3 * cap);
 
     int const i = blockIdx.x;
     int const lane = threadIdx.x;
@@ -403,10 +397,7 @@ __device__ __forceinline__ void force_backward_body(ForceArgs const& a)
                 R f, df;
                 R const r = S.P[t].w;
                 cutoff_fdf_t<CT>(cc, r, f, df);
-                bool const in = r < (R)g.rc;
-                out |= !in;
-                if (copy)
-                    S.M[t].w = in ? -0.5f * ((float)r * (float)r) : kOutside;
+                out |= !(r < (R)g.rc);
                 if (weighted)
                 {
                     R const z = (R)staged_weight(T, sStart, sCnt, t);
@@ -494,7 +485,7 @@ __device__ __forceinline__ void force_backward_body(ForceArgs const& a)
                          weighted ? 0 : uniform(sStart[g.e1]),
                          weighted ? n : uniform(sCnt[g.e1]),
                          weighted ? 0 : uniform(sStart[g.e2]),
-                         weighted ? n : uniform(sCnt[g.e2]), S.P, S.M,
+                         weighted ? n : uniform(sCnt[g.e2]), S.P,
                          S.QUEUE, grc, grc2);
         walk.run([&](int e, int count) {
             if (lane < count)

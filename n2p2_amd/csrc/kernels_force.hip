@@ -131,8 +131,7 @@ size_t force_backward_lds_bytes(ModelTables const& T, int cap, int fp32)
     size_t const r = fp32 ? sizeof(float) : sizeof(double);
     size_t b = 0;
     b += (size_t)cap * 8 * r;                     // P (4) and Q (4)
-    b += ((size_t)cap * 3 + (cap & 1)) * sizeof(double);    // ACC
-    if (!fp32 && T.narrow) b += (size_t)cap * 16;   // the search's float copy
+    b += (size_t)cap * 3 * sizeof(double);        // ACC
     b += (size_t)(T.narrow ? kPairQueueAlloc : kQueue) * sizeof(int);
     return b;
 }

@@ -205,12 +205,11 @@ void launch_fwd_r(SFArgs const& a, hipStream_t s)
 
 size_t sf_forward_lds_bytes(ModelTables const& T, int cap, int fp32)
 {
-    // Records, FP64: the search's float copy, and the pair queue or the member
-    // sums of the largest chunk.
+    // Records, and the pair queue or the member sums of the largest chunk.
     size_t const r = fp32 ? sizeof(float) : sizeof(double);
     size_t const even = (size_t)cap + (cap & 1);
     int const maxm = T.maxGroupMembers <= 8 ? 8 : 16;
-    return even * (6 * r + (!fp32 && T.narrow ? 16 : 0))
+    return even * 6 * r
          + std::max<size_t>((T.narrow ? kPairQueueAlloc : kQueue)
                             * sizeof(int), 64 * maxm * r);
 }

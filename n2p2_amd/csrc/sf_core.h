@@ -56,7 +56,6 @@ struct Stage
 {
     Vec4<R>* P;
     Vec2<R>* Q;      // null when only geometry is needed
-    Float4V* M = nullptr;   // FP64: float copy for the pair search
 };
 
 // Stages the atom's neighbours in LDS partitioned by element (stable ballot
@@ -123,7 +122,6 @@ __device__ void stage_by_element(SFArgs const& a, Stage<R> const& S, int s0,
                     p.w = (R)g.w;
                     S.P[pos] = p;
                     if (S.Q) S.Q[pos].y = R(1) / (R)g.w;
-                    if (S.M) S.M[pos] = search_entry(g);
                 }
                 start[q] += __popcll(mask);
             }
@@ -243,12 +241,9 @@ __device__ __forceinline__ void sf_forward_body(SFArgs const& a)
     Stage<R> S;
     S.P = (Vec4<R>*)sm;
     S.Q = (Vec2<R>*)(S.P + cap);
-    // The pair queue, and between groups the member sums.  FP32: after an
-    // even number of 8-byte records.
-    constexpr bool kFloat = sizeof(R) == 4;
-    bool const copy = !kFloat && HDNNP_WIDE != 1 && T.narrow;
-    S.M = copy ? (Float4V*)(S.Q + cap) : nullptr;
-    int* Q = copy ? (int*)(S.M + cap) : (int*)(S.Q + (cap + (cap & 1)));
+    // The pair queue, and between groups the member sums (16-byte aligned:
+    // after an even number of records).
+    int* Q = (int*)(S.Q + (cap + (cap & 1)));
 
     int const i = blockIdx.x;
     int const lane = threadIdx.x;
@@ -302,10 +297,7 @@ __device__ __forceinline__ void sf_forward_body(SFArgs const& a)
                 cutoff_fdf_t<CT>(cc, r, f, df);
                 if (weighted) f *= (R)staged_weight(T, sStart, sCnt, t);
                 S.Q[t].x = f;
-                bool const in = r < (R)g.rc;
-                out |= !in;
-                if (copy)
-                    S.M[t].w = in ? -0.5f * ((float)r * (float)r) : kOutside;
+                out |= !(r < (R)g.rc);
             }
             allIn = __ballot(out) == 0;
             rcCached = g.rc;
@@ -346,7 +338,7 @@ __device__ __forceinline__ void sf_forward_body(SFArgs const& a)
                              weighted ? 0 : uniform(sStart[g.e1]),
                              weighted ? n : uniform(sCnt[g.e1]),
                              weighted ? 0 : uniform(sStart[g.e2]),
-                             weighted ? n : uniform(sCnt[g.e2]), S.P, S.M, Q,
+                             weighted ? n : uniform(sCnt[g.e2]), S.P, Q,
                              grc, grc2);
             FwdMembers<R, MAXM> M;
 #pragma unroll
