@@ -18,14 +18,15 @@ namespace hdnnp {
 
 namespace {
 
-__global__ __launch_bounds__(256) void k_nn(NNArgs a, int e)
+__global__ __launch_bounds__(256) void k_nn(NNArgs a, int e,
+                                            const int* __restrict__ atoms,
+                                            int na)
 {
     int const t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= a.na[e]) return;
+    if (t >= na) return;
     ModelTables const& T = a.T;
     ElemDesc const& ed = T.elem[e];
-    int const atom = a.atoms[e][t];
-    int const na = a.na[e];
+    int const atom = atoms[t];
     int const L = ed.nlayers;
     double const* __restrict__ Gi = a.G + (size_t)atom * a.ldG;
     // scratch: value, dfdx and delta planes, each sum(width[1..L-1]) x na
@@ -640,7 +641,8 @@ hipError_t launch_nn(NNArgs& a, hipStream_t s)
 hipError_t launch_nn_atoms(NNArgs const& a, int e, hipStream_t s)
 {
     if (a.na[e] <= 0) return hipSuccess;
-    k_nn<<<(a.na[e] + 255) / 256, 256, 0, s>>>(a, e);
+    k_nn<<<(a.na[e] + 255) / 256, 256, 0, s>>>(a, e, a.atoms[e],
+                                                     a.na[e]);
     return hipGetLastError();
 }
 
