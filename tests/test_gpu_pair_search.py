@@ -93,20 +93,20 @@ def test_types_and_cutoffs(tmp_path, types, rc, cut):
     _check(tmp_path, r, elem, box, types, rc, cut)
 
 
-@pytest.mark.parametrize("cut", ["0", "1", "6"])
-def test_pairs_at_the_cutoff(tmp_path, cut):
+@pytest.mark.parametrize("cut,scale", [
+    ("1", 1.0), ("6", 1.0), ("0", 1.0 - 1e-6), ("0", 1.0 + 2e-6)])
+def test_pairs_at_the_cutoff(tmp_path, cut, scale):
     """A lattice with spacing rc / 3, moved off exactness by a few ulp: many
     pairs at rjk = rc (1 +- 1e-15), which the search lets through and the
-    evaluation has to cut off.  Cutoffs that vanish at rc and the hard one,
-    for which pairs at rounding distance may fall on either side: rc is put
-    1e-9 above the lattice distance there."""
+    evaluation has to cut off.  The hard cutoff jumps at rc, so there the pairs
+    lie 1e-6 rc inside, where all count, and 2e-6 rc outside: far above the
+    rounding of FP32 (1e-7), and within the 4e-6 rc that the search lets
+    through, so that the evaluation alone keeps them out."""
     g = np.stack(np.meshgrid(*[np.arange(5) * 2.0] * 3, indexing="ij"),
                  -1).reshape(-1, 3)
     rng = np.random.default_rng(1)
-    r = g * (1.0 + rng.uniform(-1, 1, g.shape) * 4e-16)
+    r = g * (1.0 + rng.uniform(-1, 1, g.shape) * 4e-16) * scale
     elem = rng.integers(0, 3, len(r)).astype(np.int32)
-    if cut == "0":
-        r = r * (1.0 - 1e-6)
     _check(tmp_path, r, elem, None, cut=cut)
 
 
