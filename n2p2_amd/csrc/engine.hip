@@ -1237,9 +1237,16 @@ void mdDropGraphs(hdnnp_ctx* c);
 void mdEnd(hdnnp_ctx* c)
 {
     if (!c->md.on) return;
+    auto& m = c->md;
     mdDropGraphs(c);
-    c->md.on = false;
-    c->dropList();   // the filtered list has no partner map of its own
+    m.on = false;
+    if (!c->haveNL) return;
+    // The filtered list becomes an ordinary one: the steps leave its keys
+    // unwritten and gather through the skin list's partner map.
+    c->setDevice();
+    hipCheck(launch_md_keys((int)c->n, c->dOff.p, m.skinCnt.p, m.skinKeys.p,
+                            m.newIdx.p, c->dKeys.p, c->stream), "md keys");
+    c->partnerMissing = true;
 }
 
 void mdDropGraphs(hdnnp_ctx* c)
@@ -1307,6 +1314,7 @@ void mdRebuild(hdnnp_ctx* c)
     int const n = (int)c->n;
     hipStream_t s = c->stream;
     mdDropGraphs(c);
+    c->dropList();
     hipCheck(hipMemsetAsync(m.flags.p + 4, 0, sizeof(int), s), "md flags");
     hipCheck(launch_md_wrap(n, c->dR.p, m.cell, m.flags.p + 4, s), "md wrap");
     c->hostPosValid = false;
@@ -1352,6 +1360,7 @@ void mdRebuild(hdnnp_ctx* c)
 void mdCheckStable(hdnnp_ctx* c)
 {
     if (!c->md.hFlags[2]) return;
+    c->dropList();   // not rebuilt, and its counts may be beyond the capacity
     mdEnd(c);
     throw Error(HDNNP_E_INVALID, "ERROR: MD became unstable (a coordinate "
                                  "is not finite or beyond 1e7); the time "

@@ -76,14 +76,47 @@ def test_failed_md_start(model):
     ctx.md_run(2)
 
 
-def test_end_of_md_drops_the_filtered_list(model):
-    r, elem, box = W.random_structure(300, seed=5)
+@pytest.mark.parametrize("end", ["refused list", "tuning"])
+@pytest.mark.parametrize("n", [300, 2400])
+def test_end_of_md_leaves_an_ordinary_list(model, n, end):
+    """The list of the last step, with its images and partners, after a call that
+    ends the run and builds no other one."""
+    r, elem, box = W.random_structure(n, seed=5)
     ctx = engine.Context(model)
     ctx.set_structure(r, elem, box)
-    e = ctx.evaluate(engine.FORCES_CONSISTENT)
-    ctx.md_init([10.8, 12.0, 14.0], 0.1, skin=1.0)
-    with pytest.raises(RuntimeError, match="60 periodic images"):
-        ctx.calculate_neighbor_list(70.0 * box[0, 0])    # ends the run
-    with pytest.raises(RuntimeError):
-        ctx.calculate_forces(engine.FORCES_CONSISTENT)
-    assert abs(ctx.evaluate(engine.FORCES_CONSISTENT) - e) < 1e-9 * abs(e)
+    ctx.md_init([10.8, 12.0, 14.0], 0.2, skin=1.0)
+    ctx.md_run(5)
+    x, _ = ctx.md_state()
+    if end == "tuning":
+        ctx.set_tuning(8)
+    else:
+        with pytest.raises(RuntimeError, match="60 periodic images"):
+            ctx.calculate_neighbor_list(70.0 * box[0, 0])
+    with pytest.raises(RuntimeError, match="No MD run"):
+        ctx.md_run(1)
+    ctx.calculate_symmetry_function_groups()
+    ctx.calculate_atomic_neural_networks()
+    e = ctx.calculate_energy()
+    ctx.calculate_forces(engine.FORCES_CONSISTENT)
+    got = (*ctx.neighbors(), ctx.forces())
+    ctx.set_structure(x, elem, box)
+    assert ctx.evaluate(engine.FORCES_CONSISTENT) == e
+    print("[gpu-refused]", n, end, e, flush=True)
+    for a, b in zip(got, (*ctx.neighbors(), ctx.forces())):
+        assert np.array_equal(a, b)
+
+
+def test_unstable_md_leaves_no_list(model):
+    """The step in which a coordinate runs away filtered a list that was not
+    rebuilt."""
+    r, elem, box = W.random_structure(300, seed=6)
+    v = np.zeros_like(r)
+    v[3] = 1e8
+    ctx = engine.Context(model)
+    ctx.set_structure(r, elem, box)
+    ctx.md_init([10.8, 12.0, 14.0], 0.2, skin=1.0, v=v)
+    with pytest.raises(RuntimeError, match="unstable"):
+        ctx.md_run(2)
+    for call in (ctx.calculate_symmetry_function_groups, ctx.neighbors):
+        with pytest.raises(RuntimeError, match="not calculated"):
+            call()
