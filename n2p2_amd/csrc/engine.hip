@@ -971,13 +971,15 @@ int pairRecordCap(int cap)
     return kRecordGroups + (int)std::min<int64_t>(4096, (all + 63) / 64 * 64);
 }
 
-// Atoms up to which symmetry functions without a pair record (FP64) run a block
-// per group instead of one per atom: one wave per atom leaves most wave slots
-// empty and its groups run one after another, a block per group stages the
-// neighbours again.  One per atom against one per group: 192 water atoms 43
-// and 22 us, 1,536 58 and 45, 2,304 84 and 71, 3,000 77 and 78, 5,900 146 and
-// 156; B/C/N 192 atoms 52 and 17, 1,536 72 and 56, 2,304 83 and 73, 4,500 124
-// and 146.
+// Atoms up to which symmetry functions without a pair record (FP64) run a
+// block per group instead of one per atom: one wave per atom leaves most wave
+// slots empty and its groups run one after another, a block per group stages
+// the neighbours again.  One per atom against one per group: 192 water atoms
+// 43 and 21 us, 1,500 60 and 46, 2,046 65 and 65; B/C/N 192 atoms 53 and 17,
+// 1,500 70 and 54, 2,046 71 and 70.  The line lies at eight waves per CU,
+// where both are equal.  Beyond it the kernel with one wave per atom goes by
+// the number of its rounds and either is faster (2,304 atoms 85 and 72, 86 and
+// 74; 3,000 77 and 78, 107 and 98; 4,500 128 and 123, 128 and 148).
 constexpr int kSplitAtoms = 2048;
 
 // Whether SF evaluations of this context record the passing pairs for the

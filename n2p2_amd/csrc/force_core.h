@@ -53,9 +53,13 @@
 //    order): the result does not depend on timing and repeats bit for bit.
 //    The diagonal pair order keeps the slots of a batch of 64 mostly
 //    distinct, so the adds rarely collide.
-// Bound by the LDS (six FP64 adds and four wide reads per triplet, 90% busy) in
-// FP32 and by vector instructions in FP64, where the search on the matrix
-// cores takes 196,608 water atoms from 5,230 to 5,090 us.
+// Bound in FP32 by the LDS: its unit is busy for 83% of the kernel's time on
+// 24,576 water atoms (SQ_LDS_IDX_ACTIVE per CU over SQ_BUSY_CYCLES), a third of
+// that in bank conflicts, with six scattered FP64 adds and four wide reads per
+// triplet; vector instructions take 72%.  In FP64 it is the other way round
+// (66% and 77%); the search on the matrix cores, reading the staged records
+// alone, takes 196,608 water atoms from 5,230 to 5,130 us there, with the
+// partner search running beside it.
 #ifndef HDNNP_FORCE_CORE_H
 #define HDNNP_FORCE_CORE_H
 

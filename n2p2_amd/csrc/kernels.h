@@ -200,7 +200,7 @@ hipError_t launch_energy_segments(const double* E, const int* structOff,
 // off[i] = i * slab for i <= n.
 hipError_t launch_slab_starts(int n, int slab, int* off, hipStream_t s);
 // Entries of atom i: [off[i], off[i] + cnt[i]).  order: the atoms sorted
-// by cell (processing order only).
+// by cell (processing order only), or null for their own order.
 // Partner slots of a symmetric list (nslots = slots allocated; all are
 // set to -1 first).
 hipError_t launch_nl_partner(int n, const int* off, const int* cnt,
@@ -228,8 +228,6 @@ size_t force_compact_lds_bytes(ModelTables const& T, int cap);
 size_t force_backward_lds_bytes(ModelTables const& T, int cap, int fp32);
 size_t force_list_lds_bytes(int cap, int fp32);
 
-// Entries of atom i: [off[i], off[i] + cnt[i]).  order: the atoms sorted
-// by cell (processing order only).
 // A caller-given list of n centres and M entries (idx, elem, dr: the caller's
 // arrays) as the kernels read it; stats[1..3]: largest index, some index
 // negative, some element out of range.
@@ -252,6 +250,7 @@ hipError_t launch_ext_sort(int n, int M, int nt, const int* idx,
 hipError_t launch_scatter_ext(int nt, const int64_t* srcOff, const int* src,
                               const double* cslot, const double* cself,
                               double* f, hipStream_t s);
+// Entries of atom i: [off[i], off[i] + cnt[i]).  order as launch_nl_partner.
 hipError_t launch_force_gather(int n, const int* off, const int* cnt,
                                const int* nbrJ, const int* partner,
                                const double* cslot, const double* cself,

@@ -633,10 +633,11 @@ __device__ __forceinline__ void image_range(double f, double fmin,
 // are few, and the images of a cell below three cutoffs overflow their
 // staging, which then cost a count and a fill by the per-atom kernels.  List
 // builds including the host's wait, cells against this: 192 water atoms (27
-// images) 292 -> 62 us, 1,536 225 -> 100 us, 1,000 B/C/N atoms 202 -> 84 us.
-// The work grows as n^2: 2,000 B/C/N atoms take 123 us against the cells'
-// 131, 4,000 230 against 131 (water, wider cutoff: 129 against 168 and 200
-// against 182), hence the bound of 2,048.
+// images) 253 -> 64 us, 1,500 218 -> 99 us, 1,002 B/C/N atoms 145 -> 83 us.
+// The work grows as n^2: 2,046 atoms take 113 us against the cells' 143 (water,
+// B/C/N 123 against 144), 2,304 128 against 146 and 140 against 121, 3,600 182
+// against 153 and 209 against 138, hence the bound of 2,048, below which it is
+// the faster form for both.
 template <int MODE>
 __global__ __launch_bounds__(64) void k_nl_batch(
     int n, double rc2, double rcm, const double* __restrict__ r,
@@ -831,7 +832,8 @@ __global__ void k_slab_starts(int n, int slab, int* __restrict__ off)
 // atom i are the tail of its list from the first key with j >= i, so the
 // lanes work on that range only.  Slots left unwritten (an inconsistent
 // list) keep the -1 the launcher fills in.  One wave per atom, atoms in
-// cell order (order = atoms sorted by cell) with the XCD-aware mapping: the
+// cell order (order = atoms sorted by cell; null: their own order, in lists
+// without cells) with the XCD-aware mapping: the
 // lists searched by neighbouring atoms overlap and stay in one L2.
 __global__ __launch_bounds__(64) void k_partner(
     int n, const int* __restrict__ off, const int* __restrict__ cnt,

@@ -28,12 +28,13 @@
 //      exponential and (eta, rs, lambda) runs sorted by zeta sharing one
 //      chain of powers of plambda (PowChain, bit-identical to pow_int);
 //   5. member sums are reduced through LDS in a fixed order (deterministic).
-// Bound by the issue of instructions (vector and scalar together; LDS and
-// memory are below 20%).  With the search on the matrix cores, the sums
-// through LDS and wide pairs straight to the lanes: 196,608 water atoms 2,190
-// -> 1,950 us in FP32 (1,716 us without the partner search beside it) and
-// 4,370 -> 3,970 us in FP64; 512 B/C/N structures (wide type only) 1,820 ->
-// 1,355 us.
+// Bound by the issue of vector instructions: on 24,576 water atoms a wave
+// issues 6,810 of them (FP32; 9,980 in FP64), which at four cycles each is all
+// of the kernel's time for a SIMD's 24 waves (FP64 82%); the LDS unit is busy
+// for 38% of it (41%).  With the search on the matrix cores, the sums through
+// LDS and wide pairs straight to the lanes: 196,608 water atoms 2,190 -> 1,830
+// us in FP32 and 4,370 -> 3,730 us in FP64; 512 B/C/N structures (wide type
+// only) 1,820 -> 1,280 us.
 #ifndef HDNNP_SF_CORE_H
 #define HDNNP_SF_CORE_H
 
@@ -227,7 +228,8 @@ __device__ __forceinline__ void triplet_forward(
 #endif
 }
 
-// Body of the forward kernel (one 64-lane workgroup per atom).
+// Body of the forward kernel: one 64-lane workgroup per atom, or per atom and
+// group (SFArgs::parts).
 template <int MAXM, int CT, bool GENPOW, typename R>
 __device__ __forceinline__ void sf_forward_body(SFArgs const& a)
 {
