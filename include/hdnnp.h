@@ -223,7 +223,9 @@ int hdnnp_set_positions_device(hdnnp_ctx* c, const double* r_device);
 /* Structure::calculateNeighborList(cutoff, false) (Structure.cpp:287-399):
  * per atom all (j, image) with |r_i - r_j + image| <= cutoff, ordered by j
  * then image components ascending; bit-identical index, d and dr.
- * Built with a cell list on the device. */
+ * Built on the device, by cells or (small structures) without.  A cutoff the
+ * checks refuse (60 images, number of cells) leaves the list before; a build
+ * that fails later leaves none. */
 int hdnnp_neighbor_list(hdnnp_ctx* c, double cutoff);
 /* Mode::calculateSymmetryFunctionGroups(structure, derivatives)
  * (Mode.cpp:1561-1640).  Computes the scaled SF values G.  With
@@ -298,7 +300,8 @@ int hdnnp_set_neighbor_list(hdnnp_ctx* c, int64_t ncentre,
 /* InterfaceLammps::getForces (InterfaceLammps.cpp:546-581) after
  * hdnnp_forces on a caller-given list: adds every centre's self force to
  * f[centre_index] and every entry's pair force to f[nbr_index] (f has nout
- * rows of 3, internal units), centres in order, entries in list order. */
+ * rows of 3, internal units), centres in order, entries in list order.  An
+ * error before the forces of this list are computed. */
 int hdnnp_get_scattered_forces(hdnnp_ctx* c, int64_t nout, double* f);
 /* No counterpart in the reference.  hdnnp_get_scattered_forces for callers
  * that cannot allocate device memory (code under HIP graph capture, tight
