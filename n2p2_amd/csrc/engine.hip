@@ -1611,6 +1611,8 @@ void hdnnp_ctx_destroy(hdnnp_ctx* c)
     c->dEnergy.release(); c->dStatOut.release(); c->dEw.release();
     c->dStructOf.release(); c->dStructOff.release(); c->dCells.release();
     c->dEnergySeg.release();
+    c->dPairs.release();
+    c->dScatOff.release(); c->dScatSrc.release(); c->dScatF.release();
     mdDropGraphs(c);
     {
         auto& m = c->md;
