@@ -335,8 +335,10 @@ const double* hdnnp_forces_device(hdnnp_ctx* c);
  * caller's units (eV/A/amu with dt in fs: 9.648533212e-3), initial
  * velocities v (n x 3, NULL = zero), force mode (HDNNP_FORCES_*).  It
  * computes the forces at the initial positions.  hdnnp_set_structure,
- * hdnnp_set_positions*, hdnnp_neighbor_list, hdnnp_evaluate and
- * hdnnp_set_neighbor_list end the run. */
+ * hdnnp_set_positions*, hdnnp_neighbor_list, hdnnp_evaluate,
+ * hdnnp_set_neighbor_list, hdnnp_train_gradient and a change of the launch
+ * forms end the run; where the call builds no other list, that of the last
+ * step stays in use.  A run whose list rebuild failed takes no more steps. */
 int hdnnp_md_init(hdnnp_ctx* c, const double* masses, double dt, double skin,
                   double ftoa, const double* v, int force_mode, int use_graph);
 /* nsteps steps.  epot[k] (the model's energy) and ekin[k] = sum m v^2 / 2
