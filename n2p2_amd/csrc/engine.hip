@@ -1322,6 +1322,7 @@ void mdRebuild(hdnnp_ctx* c)
     c->hostPosValid = false;
     buildNeighborList(c, m.rc + m.skin);
     c->waitPartner();   // before any graph is captured on the main stream
+    c->dropList();      // the skin list becomes the run's; filtered below
     std::swap(c->dKeys, m.skinKeys);
     std::swap(c->dPartner, m.skinPartner);
     std::swap(c->dCount, m.skinCnt);
@@ -1354,6 +1355,7 @@ void mdRebuild(hdnnp_ctx* c)
         c->dPairs.ensure(std::max<size_t>(
             (size_t)n * (size_t)pairRecordCap(m.cap), 1));
     c->Mvalid = false;
+    c->haveNL = true;
     m.rebuilds += 1;
 }
 
